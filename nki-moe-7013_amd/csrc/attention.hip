@@ -110,10 +110,6 @@ __device__ __forceinline__ void qkv_finish_head(
 // arithmetic per element as qkv_finish_head; the sum of squares runs in the
 // wave's reduction order.
 constexpr int QKV_DEC_MAX_T = 16;
-#ifndef QMOE_QKV_PIPE_MIN_T
-#define QMOE_QKV_PIPE_MIN_T 256
-#endif
-constexpr int QKV_PIPE_MIN_T = QMOE_QKV_PIPE_MIN_T;  // token rows from which the 256-row pipeline is used
 
 // One head row of the decode finish, lane l holding elements l and l + 64
 // (its RoPE partner): RMSNorm over the 128 values (one wave reduction), the
@@ -1275,7 +1271,10 @@ extern "C" int qmoe_qkv_norm_rope(const qmoe_bf16* x, const qmoe_bf16* wqkv,
       T * H * 2 < (1ll << 31) && (Hq + 2 * Hkv) * HD * H * 2 < (1ll << 31))
     return qkv_wide_launch(x, wqkv, q_norm_w, k_norm_w, rope_cos, rope_sin, positions, T, S, H, Hq, Hkv, S_max,
                            max_p, eps, q_out, k_cache, v_cache, as_stream(stream));
-  if (T >= QKV_PIPE_MIN_T && H % 64 == 0 && T * H * 2 < (1ll << 32)) {
+  // The direct-to-LDS pipelines take every other row count (17 to 255 rows,
+  // which the register-staged 128 x 128 tiles ran in 55-60 us, take 17-20 us on
+  // the 64-row tiles); the register-staged kernel keeps x of 4 GiB and more.
+  if (T * H * 2 < (1ll << 32)) {
     // 256-row tiles once they give every CU a workgroup; below that 128-row
     // tiles, two per CU, while they fill the CUs.  Fewer tiles than CUs: one
     // workgroup per CU with four stages in flight, 64-row tiles while those

@@ -338,6 +338,86 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_pk_kernel(const uint16_t* __r
   }
 }
 
+// Skinny GEMM for 9 <= M <= 64 rows of A (larger decode batches, short
+// prompts): gemv_pk_kernel's weight stream (K = 512 * WAVES, one 1 KB LDS-DMA
+// per weight row and wave, NB columns per workgroup) with whole 16-row A
+// fragments.  The weights stay in LDS while the MT = ceil(M / 16) row tiles
+// pass over them; a tile's 16 fragments (8 k-values of 16 rows each) come
+// straight from global memory, the next tile's in flight behind this one's
+// MFMAs.  Bound by the weight stream plus the A rows that every workgroup
+// re-reads from L2 (M * K * 2 bytes, 1-4 us of a CU's L2 port).
+template <int WAVES, int NB, int MT, int MODE>
+__global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(const uint16_t* __restrict__ A, int64_t lda,
+                                                                 const uint16_t* __restrict__ B, int M, int N,
+                                                                 int K, void* __restrict__ C, int64_t ldc) {
+  constexpr int NT = (NB + 15) / 16;  // 16-column MFMA tiles
+  constexpr int RLD = NB + 1;
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];  // weights; then the partials
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int n0 = blockIdx.x * NB;
+  const int kw = wave * 512;
+  const int col = lane & 15, kg = lane >> 4;
+  uint8_t* wl = smem + wave * (NB * GV_ROWB);
+  u32x4 af[2][16];
+  auto load_a = [&](u32x4 (&dst)[16], int mt) {  // rows past M repeat the last one; their products are not stored
+    const uint16_t* p = A + int64_t(min(mt * 16 + col, M - 1)) * lda + kw + kg * 8;
+#pragma unroll
+    for (int s = 0; s < 16; ++s) dst[s] = ld16(p + s * 32);
+  };
+  load_a(af[0], 0);
+  {
+    const pipe::i32x4 rb = pipe::make_rsrc(B, uint32_t(int64_t(N) * K * 2));
+    const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>(wl));
+#pragma unroll
+    for (int r = 0; r < NB; ++r) {
+      const uint32_t off = n0 + r < N ? uint32_t((int64_t(n0 + r) * K + kw) * 2) + lane * 16u : pipe::PAD;
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds"
+                   :
+                   : "s"(lds0 + uint32_t(r * GV_ROWB)), "v"(off), "s"(rb)
+                   : "memory");
+    }
+  }
+  pipe::wait_vm<0>();  // this wave's weight rows are in LDS (and its first A tile in registers)
+  f32x4 acc[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{};
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    if (i + 1 < MT) load_a(af[(i + 1) & 1], i + 1);
+#pragma unroll
+    for (int s = 0; s < 16; ++s)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const u32x4 b = *reinterpret_cast<const u32x4*>(wl + min(j * 16 + col, NB - 1) * GV_ROWB + kg * 16 + s * 64);
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, af[i & 1][s]),
+                                                            __builtin_bit_cast(bf16x8, b), acc[i][j], 0, 0, 0);
+      }
+  }
+  // lane l holds column l % 16 of tile j, rows 16 i + (l / 16) * 4 + 0..3
+  __syncthreads();  // the weights are used up: their LDS takes the partials
+  float* red = reinterpret_cast<float*>(smem);  // [WAVES][MT * 16][RLD]
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+      if (j * 16 + col < NB)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) red[(wave * MT * 16 + i * 16 + kg * 4 + e) * RLD + j * 16 + col] = acc[i][j][e];
+  __syncthreads();
+  for (int i = t; i < min(M, MT * 16) * NB; i += 64 * WAVES) {
+    const int m = i / NB, n = i % NB;
+    if (n0 + n < N) {
+      float v = red[m * RLD + n];
+#pragma unroll
+      for (int w = 1; w < WAVES; ++w) v += red[(w * MT * 16 + m) * RLD + n];
+      store_out<MODE>(C, int64_t(m) * ldc + n0 + n, v);
+    }
+  }
+}
+
 // ------------------------------------------------------------------ MFMA tile
 // Grid = every (row tile, column tile) pair, renumbered XCD-contiguously and
 // then walked in groups of 8 row tiles per column sweep, so the workgroups
@@ -642,8 +722,88 @@ __global__ __launch_bounds__(256, OCC) void gemm_splitk_kernel(const uint16_t* _
     }
 }
 
+// The slices of a 17 <= M <= 64 row problem (decode-batch o_proj): workgroup
+// (64 columns, 512 k-values) copies its weight rows and the A rows' slice
+// into LDS in one go (1 KB LDS-DMA per row: whole lines, everything requested
+// at once), then 8 waves run the 16 x 16 tiles.  One memory round trip long:
+// splitting K keeps the A bytes per workgroup at M KB, where a workgroup that
+// owns whole columns re-reads all of A (M * K * 2 bytes at the 16-row fragment
+// loads' 16 B per clock: 2048 x 4096 takes 10.9 us at 32 rows, 18.2 at 64).
+constexpr int SL_K = 512, SL_N = 64;
+template <int MT>
+__global__ __launch_bounds__(512) void gemm_slice_kernel(const uint16_t* __restrict__ A, int64_t lda,
+                                                         const uint16_t* __restrict__ B, int M, int N, int K,
+                                                         float* __restrict__ part) {
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];  // SL_N weight rows, then 16 MT A rows
+  const int splits = K / SL_K, slice = int(blockIdx.x) % splits, n0 = int(blockIdx.x) / splits * SL_N;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const pipe::i32x4 ra = pipe::make_rsrc(A, uint32_t((int64_t(M) - 1) * lda * 2 + int64_t(K) * 2));
+  const pipe::i32x4 rb = pipe::make_rsrc(B, uint32_t(int64_t(N) * K * 2));
+  const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>(smem));
+  const uint32_t kb = uint32_t(slice) * SL_K * 2 + lane * 16u;
+#pragma unroll
+  for (int i = 0; i < SL_N / 8; ++i) {
+    const int r = wave * (SL_N / 8) + i;
+    const uint32_t off = n0 + r < N ? uint32_t(int64_t(n0 + r) * K * 2) + kb : pipe::PAD;
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds"
+                 :
+                 : "s"(lds0 + uint32_t(r * GV_ROWB)), "v"(off), "s"(rb)
+                 : "memory");
+  }
+#pragma unroll
+  for (int i = 0; i < 2 * MT; ++i) {
+    const int r = wave * 2 * MT + i;
+    pipe::dma16(lds0 + uint32_t((SL_N + r) * GV_ROWB), r < M ? uint32_t(int64_t(r) * lda * 2) + kb : pipe::PAD, ra, 0);
+  }
+  pipe::wait_vm<0>();
+  __syncthreads();
+  const int col = lane & 15, kg = lane >> 4, ct = wave & 3;
+  const uint8_t* bp = smem + (ct * 16 + col) * GV_ROWB + kg * 16;
+  float* dst = part + int64_t(slice) * M * N;
+  for (int mt = wave >> 2; mt < MT; mt += 2) {
+    const uint8_t* ap = smem + (SL_N + mt * 16 + col) * GV_ROWB + kg * 16;
+    f32x4 acc[2] = {f32x4{}, f32x4{}};
+#pragma unroll
+    for (int s = 0; s < SL_K / 32; ++s)
+      acc[s & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(ap + s * 64),
+                                                           *reinterpret_cast<const bf16x8*>(bp + s * 64), acc[s & 1],
+                                                           0, 0, 0);
+    const int n = n0 + ct * 16 + col;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int m = mt * 16 + kg * 4 + e;
+      if (m < M && n < N) dst[int64_t(m) * N + n] = acc[0][e] + acc[1][e];
+    }
+  }
+}
+
+// Sum of the slices' float4 at float offset o, in slice order; with S known
+// every load is in flight at once (S = 0: any count).
+template <int S>
+__device__ __forceinline__ float4 sum_slices(const float* __restrict__ part, int splits, int64_t slab, int64_t o) {
+  const int n = S ? S : splits;
+  float4 v[S ? S : 1];
+  if constexpr (S > 0) {
+#pragma unroll
+    for (int s = 0; s < S; ++s) v[s] = *reinterpret_cast<const float4*>(part + s * slab + o);
+  } else {
+    v[0] = *reinterpret_cast<const float4*>(part + o);
+  }
+  float4 a = v[0];
+#pragma unroll
+  for (int s = 1; s < n; ++s) {
+    const float4 w = S ? v[S ? s : 0] : *reinterpret_cast<const float4*>(part + s * slab + o);
+    a.x += w.x;
+    a.y += w.y;
+    a.z += w.z;
+    a.w += w.w;
+  }
+  return a;
+}
+
 // C (mode) = sum over slices in order; 4 consecutive columns per thread.
-template <int MODE>
+template <int MODE, int S>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ part, int splits, int M,
                                                            int N, void* C, int64_t ldc) {
   const int64_t q = int64_t(blockIdx.x) * 256 + threadIdx.x;  // float4 index
@@ -651,14 +811,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
   if (q >= int64_t(M) * per_row) return;
   const int64_t row = q / per_row, col = (q - row * per_row) * 4;
   const int64_t slab = int64_t(M) * N;
-  float4 v = *reinterpret_cast<const float4*>(part + row * N + col);
-  for (int s = 1; s < splits; ++s) {
-    const float4 w = *reinterpret_cast<const float4*>(part + s * slab + row * N + col);
-    v.x += w.x;
-    v.y += w.y;
-    v.z += w.z;
-    v.w += w.w;
-  }
+  const float4 v = sum_slices<S>(part, splits, slab, row * N + col);
   store_out<MODE>(C, row * ldc + col, v.x);
   store_out<MODE>(C, row * ldc + col + 1, v.y);
   store_out<MODE>(C, row * ldc + col + 2, v.z);
@@ -668,6 +821,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
 // The ADD_F32 reduction of whole rows (one workgroup per row, the chunks of
 // norm_impl.hpp) followed by the row's RMSNorm: C[row] += sum of the slices
 // (splitk_reduce_kernel's order), x_out[row] = bf16(rms_w * C[row] * r).
+template <int S>
 __global__ __launch_bounds__(NORM_THREADS) void splitk_reduce_norm_kernel(
     const float* __restrict__ part, int splits, int M, int N, float* C, const uint16_t* __restrict__ rms_w,
     float eps, uint16_t* __restrict__ x_out) {
@@ -681,15 +835,8 @@ __global__ __launch_bounds__(NORM_THREADS) void splitk_reduce_norm_kernel(
     const int c = int(threadIdx.x) + j * NORM_THREADS;
     if (c < nchunk) {
       const int64_t o = row * N + 4 * c;
-      float4 a = *reinterpret_cast<const float4*>(part + o);
-      for (int s = 1; s < splits; ++s) {
-        const float4 w = *reinterpret_cast<const float4*>(part + s * slab + o);
-        a.x += w.x;
-        a.y += w.y;
-        a.z += w.z;
-        a.w += w.w;
-      }
       float4 h = *reinterpret_cast<const float4*>(C + o);
+      const float4 a = sum_slices<S>(part, splits, slab, o);
       h.x += a.x;
       h.y += a.y;
       h.z += a.z;
@@ -739,6 +886,56 @@ static int splitk_plan(int64_t M, int64_t N, int64_t K, SplitTile* tile) {
   return splits > 1 ? splits : 0;
 }
 
+// The sum of the slices into C (mode), with x_out (ADD_F32, rows of N floats)
+// followed by the rows' RMSNorm.
+template <int MODE, int S>
+static int launch_reduce_s(const float* part, int splits, int M, int N, void* C, int64_t ldc, hipStream_t s,
+                           const uint16_t* rms_w, float eps, uint16_t* x_out) {
+  if (x_out) {
+    hipLaunchKernelGGL(splitk_reduce_norm_kernel<S>, dim3(unsigned(M)), dim3(NORM_THREADS), 0, s, part, splits, M, N,
+                       static_cast<float*>(C), rms_w, eps, x_out);
+    return hip_status("qmoe_gemm_ws(reduce + norm)");
+  }
+  const int64_t n4 = int64_t(M) * (N / 4);
+  hipLaunchKernelGGL((splitk_reduce_kernel<MODE, S>), dim3(unsigned((n4 + 255) / 256)), dim3(256), 0, s, part, splits,
+                     M, N, C, ldc);
+  return hip_status("qmoe_gemm_ws(reduce)");
+}
+
+template <int MODE>
+static int launch_reduce(const float* part, int splits, int M, int N, void* C, int64_t ldc, hipStream_t s,
+                         const uint16_t* rms_w, float eps, uint16_t* x_out) {
+  switch (splits) {
+    case 2: return launch_reduce_s<MODE, 2>(part, splits, M, N, C, ldc, s, rms_w, eps, x_out);
+    case 4: return launch_reduce_s<MODE, 4>(part, splits, M, N, C, ldc, s, rms_w, eps, x_out);
+    case 8: return launch_reduce_s<MODE, 8>(part, splits, M, N, C, ldc, s, rms_w, eps, x_out);
+    default: return launch_reduce_s<MODE, 0>(part, splits, M, N, C, ldc, s, rms_w, eps, x_out);
+  }
+}
+
+// gemm_slice_kernel takes a split-K plan whose slices are its 512 columns,
+// while its workgroups fit the CUs in one round.  o_proj into the residual
+// with the norm (N = 2048, K = 4096; 17 / 32 / 64 rows, reduction included):
+// 18.1 / 18.2 / 19.2 us on 128 x 128 tiles, 10.2 / 10.6 / 12.9 us here; with
+// 1.25 rounds (N = 5120, K = 2048) 13.4 us against 10.9.
+static bool slice_ok(int64_t M, int64_t N, int64_t K, int splits) {
+  return M >= 17 && M <= 64 && splits * SL_K == K && (N + SL_N - 1) / SL_N * splits <= current_device_cus();
+}
+
+template <int MT>
+static void launch_slices(const uint16_t* A, int64_t lda, const uint16_t* B, int M, int N, int K, float* part,
+                          hipStream_t s) {
+  constexpr int SMEM = (SL_N + 16 * MT) * GV_ROWB;
+  static const bool attr = [] {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_slice_kernel<MT>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, SMEM);
+    return true;
+  }();
+  (void)attr;
+  hipLaunchKernelGGL(gemm_slice_kernel<MT>, dim3(unsigned((N + SL_N - 1) / SL_N * (K / SL_K))), dim3(512), SMEM, s, A,
+                     lda, B, M, N, K, part);
+}
+
 template <class P, int MODE>
 static int launch_splitk(const uint16_t* A, int64_t lda, const uint16_t* B, int M, int N, int K, int splits,
                          float* part, void* C, int64_t ldc, hipStream_t s, const uint16_t* rms_w = nullptr,
@@ -749,19 +946,20 @@ static int launch_splitk(const uint16_t* A, int64_t lda, const uint16_t* B, int 
     return true;
   }();
   (void)attr;
-  const int64_t tiles = int64_t((M + P::BM - 1) / P::BM) * ((N + P::BN - 1) / P::BN);
-  hipLaunchKernelGGL((gemm_splitk_kernel<P, 2>), dim3(unsigned(tiles * splits)), dim3(256), P::SMEM, s, A, lda,
-                     B, M, N, K, splits, part);
-  if (int rc = hip_status("qmoe_gemm_ws(slices)")) return rc;
-  if (x_out) {  // ADD_F32 into rows of N floats, then their RMSNorm
-    hipLaunchKernelGGL(splitk_reduce_norm_kernel, dim3(unsigned(M)), dim3(NORM_THREADS), 0, s, part, splits, M, N,
-                       static_cast<float*>(C), rms_w, eps, x_out);
-    return hip_status("qmoe_gemm_ws(reduce + norm)");
+  if (slice_ok(M, N, K, splits)) {
+    if (M <= 32)
+      launch_slices<2>(A, lda, B, M, N, K, part, s);
+    else if (M <= 48)
+      launch_slices<3>(A, lda, B, M, N, K, part, s);
+    else
+      launch_slices<4>(A, lda, B, M, N, K, part, s);
+  } else {
+    const int64_t tiles = int64_t((M + P::BM - 1) / P::BM) * ((N + P::BN - 1) / P::BN);
+    hipLaunchKernelGGL((gemm_splitk_kernel<P, 2>), dim3(unsigned(tiles * splits)), dim3(256), P::SMEM, s, A, lda,
+                       B, M, N, K, splits, part);
   }
-  const int64_t n4 = int64_t(M) * (N / 4);
-  hipLaunchKernelGGL(splitk_reduce_kernel<MODE>, dim3(unsigned((n4 + 255) / 256)), dim3(256), 0, s, part, splits,
-                     M, N, C, ldc);
-  return hip_status("qmoe_gemm_ws(reduce)");
+  if (int rc = hip_status("qmoe_gemm_ws(slices)")) return rc;
+  return launch_reduce<MODE>(part, splits, M, N, C, ldc, s, rms_w, eps, x_out);
 }
 
 int64_t gemm_splitk_bytes(int64_t M, int64_t N, int64_t K) {
@@ -905,6 +1103,60 @@ static int launch_gemv_pk(const uint16_t* A, int64_t lda, const uint16_t* B, int
   return fail(QMOE_ERR_INVALID, "qmoe_gemm: packed GEMV needs K in {512, 1024, 2048, 4096}");
 }
 
+// Rows and shapes that gemm_skinny_kernel takes: up to two rounds of its
+// 20-column workgroups.  Measured against the kernels that took these shapes
+// before (16-row GEMV, 64 x 64 tiles), 9 / 16 / 32 / 64 rows: N = 5120, K =
+// 2048 8.9 / 11.5 / 12.1 / 13.0 -> 6.2 / 6.9 / 8.8 / 12.5 us; N = 2048, K =
+// 4096 20.5 / 20.8 / 21.8 / 23.1 -> 6.5 / 7.8 / 10.9 / 18.2 us.  At the
+// vocabulary's N = 151936 every one of 7597 workgroups re-reads A and the
+// tiles stay ahead (135 / 169 / 179 us against 148 / 222 / 314 at 12 / 32 / 64).
+static bool skinny_ok(int64_t M, int64_t N, int64_t K) {
+  return M >= 9 && M <= 64 && (K == 512 || K == 1024 || K == 2048 || K == 4096) && N * K * 2 < (1ll << 31) &&
+         N <= 40ll * current_device_cus();
+}
+
+template <int WAVES, int NB, int MT, int MODE>
+static int launch_skinny_t(const uint16_t* A, int64_t lda, const uint16_t* B, int M, int N, int K, void* C,
+                           int64_t ldc, hipStream_t s) {
+  constexpr int W_BYTES = WAVES * NB * GV_ROWB, R_BYTES = WAVES * MT * 16 * (NB + 1) * 4;
+  constexpr int SMEM = W_BYTES > R_BYTES ? W_BYTES : R_BYTES;
+  static_assert(SMEM <= 160 * 1024, "LDS");
+  static const bool attr = [] {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_skinny_kernel<WAVES, NB, MT, MODE>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, SMEM);
+    return true;
+  }();
+  (void)attr;
+  hipLaunchKernelGGL((gemm_skinny_kernel<WAVES, NB, MT, MODE>), dim3(unsigned((N + NB - 1) / NB)), dim3(64 * WAVES),
+                     SMEM, s, A, lda, B, M, N, K, C, ldc);
+  return hip_status("qmoe_gemm(skinny)");
+}
+
+template <int MODE>
+static int launch_skinny(const uint16_t* A, int64_t lda, const uint16_t* B, int M, int N, int K, void* C,
+                         int64_t ldc, hipStream_t s) {
+  // columns per workgroup by the rule of the packed GEMV
+  const int cus = current_device_cus();
+  const int nb = N >= 20 * cus && K <= 2048 ? 20 : N >= 16 * cus ? 16 : N >= 8 * cus ? 8 : 4;
+#define QMOE_SK(W, NB_)                                                                            \
+  if (K == 512 * W && nb == NB_)                                                                   \
+    return M <= 16   ? launch_skinny_t<W, NB_, 1, MODE>(A, lda, B, M, N, K, C, ldc, s)              \
+           : M <= 32 ? launch_skinny_t<W, NB_, 2, MODE>(A, lda, B, M, N, K, C, ldc, s)              \
+           : M <= 48 ? launch_skinny_t<W, NB_, 3, MODE>(A, lda, B, M, N, K, C, ldc, s)              \
+                     : launch_skinny_t<W, NB_, 4, MODE>(A, lda, B, M, N, K, C, ldc, s);
+#define QMOE_SK_W(W) QMOE_SK(W, 4) QMOE_SK(W, 8) QMOE_SK(W, 16)
+  QMOE_SK_W(1)
+  QMOE_SK_W(2)
+  QMOE_SK_W(4)
+  QMOE_SK_W(8)
+  QMOE_SK(1, 20)
+  QMOE_SK(2, 20)
+  QMOE_SK(4, 20)
+#undef QMOE_SK_W
+#undef QMOE_SK
+  return fail(QMOE_ERR_INVALID, "qmoe_gemm: skinny GEMM needs K in {512, 1024, 2048, 4096}");
+}
+
 template <int MODE>
 static int launch_gemv(const uint16_t* A, int64_t lda, const uint16_t* B, int M, int N, int K,
                        void* C, int64_t ldc, hipStream_t s) {
@@ -954,6 +1206,16 @@ int gemm_launch(const uint16_t* A, int64_t lda, const uint16_t* B, int64_t M, in
   QMOE_REQUIRE(lda % 8 == 0, "qmoe_gemm: lda must be a multiple of 8");
   QMOE_REQUIRE(M < (1ll << 31) && N < (1ll << 31) && K < (1ll << 31), "qmoe_gemm: dims overflow");
   if (M == 0) return QMOE_OK;
+  if (skinny_ok(M, N, K) && (M - 1) * lda * 2 + K * 2 < (1ll << 31)) {
+    switch (mode) {
+      case QMOE_GEMM_STORE_BF16:
+        return launch_skinny<QMOE_GEMM_STORE_BF16>(A, lda, B, int(M), int(N), int(K), C, ldc, s);
+      case QMOE_GEMM_STORE_F32:
+        return launch_skinny<QMOE_GEMM_STORE_F32>(A, lda, B, int(M), int(N), int(K), C, ldc, s);
+      default:
+        return launch_skinny<QMOE_GEMM_ADD_F32>(A, lda, B, int(M), int(N), int(K), C, ldc, s);
+    }
+  }
   if (M <= 16 && M * K <= 32768) {
     QMOE_REQUIRE(K % 512 == 0, "qmoe_gemm: gemv path needs K %% 512 == 0 (K=%lld)", (long long)K);
     switch (mode) {

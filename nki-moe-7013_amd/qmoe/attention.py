@@ -25,6 +25,10 @@ def rope_tables(head_dim: int, max_pos: int, theta: float, device) -> tuple:
     return freqs.cos().contiguous(), freqs.sin().contiguous()
 
 
+# Decode batches of up to this many rows take the skinny projection GEMM into
+# fp32 and finish q/k/v inside the attention launch.
+FUSED_DECODE_MAX_ROWS = 64
+
 # Chunks of up to this many query rows at a device-held start run as
 # single-query decode problems (qmoe_attn_decode_chunk).
 CHUNK_DECODE_MAX = 16
@@ -102,7 +106,7 @@ class Attention:
         int, or an int32 ``[1]`` device tensor for graph replays at any position).
         S == 1: decode; row b sees cache entries ``[0, positions[b]]`` (at most
         the first ``max_ctx`` when a context bucket is given), on every path.
-        On the GEMV path (B <= 16 decode rows) the finish runs inside the
+        Up to ``FUSED_DECODE_MAX_ROWS`` decode rows the finish runs inside the
         attention launch (``attn_decode_fused``).
         ``norm = (rms_w, eps)``: ``x`` is the fp32 residual row itself (B*S == 1)
         and the input RMSNorm is fused into the QKV GEMV.
@@ -111,15 +115,18 @@ class Attention:
         (instead of the residual itself).
         """
         n_ws = ops.qkv_norm_rope_workspace(B * S, x.shape[1], self.n_q, self.n_kv, self.head_dim)
+        n_raw = n_ws
+        if S == 1 and n_ws == 0 and 0 < B <= FUSED_DECODE_MAX_ROWS and x.shape[1] in ops.SKINNY_K:
+            n_raw = B * self.wqkv.shape[0] * 4
         qws = self._ws.get(("qkv", B * S))
-        if qws is None:
-            qws = torch.empty(max(n_ws // 4, 1), dtype=torch.float32, device=x.device)
+        if qws is None or qws.numel() * 4 < n_raw:
+            qws = torch.empty(max(n_raw // 4, 1), dtype=torch.float32, device=x.device)
             self._ws[("qkv", B * S)] = qws
         if norm is not None and (B * S != 1 or n_ws == 0):
             raise ValueError("the fused input norm takes one fp32 row on the GEMV path")
-        if S == 1 and n_ws > 0:
-            # decode on the GEMV path: raw projection, then finish + attention in one launch
-            raw = qws[: n_ws // 4].view(B, -1)
+        if S == 1 and n_raw > 0:
+            # decode: raw projection, then finish + attention in one launch
+            raw = qws[: n_raw // 4].view(B, -1)
             if norm is not None:
                 ops.gemv_rmsnorm(x, norm[0], norm[1], self.wqkv, _lib.GEMM_STORE_F32, out=raw)
             else:

@@ -420,6 +420,10 @@ def moe_combine(
 
 
 # ----------------------------------------------------------------- GEMM
+# Reduction lengths of the GEMV and skinny (up to 64 rows) GEMM kernels.
+SKINNY_K = (512, 1024, 2048, 4096)
+
+
 def gemm_workspace(M: int, N: int, K: int, device) -> Optional[torch.Tensor]:
     """Workspace for :func:`gemm` with split-K (``None`` when the shape is
     not split: it already fills the GPU)."""

@@ -1,0 +1,108 @@
+"""Batched-decode sizes (9 to 64 rows): the skinny and sliced GEMMs, the QKV
+projection of short prompts, and the fused decode attention layer."""
+
+import pytest
+import torch
+
+import oracle
+from gpu_util import announce, assert_close_layer, bf16_randn
+from qmoe import _lib, ops
+from qmoe.attention import Attention, KVCache, rope_tables
+
+pytestmark = pytest.mark.gpu
+
+H, HQ, HKV, D = 2048, 32, 4, 128
+
+
+def _gen(dev, seed):
+    return torch.Generator(device=dev).manual_seed(seed)
+
+
+# every row-tile count and its edges; column remainders of the 4-, 8-, 16- and
+# 20-column workgroups and of the 64-column slices; every K
+@pytest.mark.parametrize("M", [9, 16, 17, 32, 33, 48, 49, 64])
+@pytest.mark.parametrize("N,K", [(5120, 2048), (2048, 4096), (1111, 512), (4133, 1024), (5129, 1024), (64, 2048)])
+def test_skinny_gemm(dev, M, N, K):
+    announce(f"skinny gemm M={M} N={N} K={K}")
+    g = _gen(dev, M * 7 + N)
+    A = bf16_randn((M, K), g, dev)
+    B = bf16_randn((N, K), g, dev, std=0.05)
+    base = torch.randn(M, N, generator=g, device=dev)
+    ref = A.double() @ B.double().t()
+    # fp32 sums of K products in any order: K * 2^-24 of the sum of magnitudes
+    bound = (A.double().abs() @ B.double().abs().t()) * (K * 2.0 ** -24)
+    ws = ops.gemm_workspace(M, N, K, dev)
+    for w in (None, ws) if ws is not None else (None,):
+        c = ops.gemm(A, B, _lib.GEMM_STORE_F32, workspace=w)
+        again = ops.gemm(A, B, _lib.GEMM_STORE_F32, workspace=w)
+        cb = ops.gemm(A, B, _lib.GEMM_STORE_BF16, workspace=w)
+        acc = base.clone()
+        ops.gemm(A, B, _lib.GEMM_ADD_F32, out=acc, workspace=w)
+        torch.cuda.synchronize()
+        assert bool(((c.double() - ref).abs() <= bound).all())
+        assert torch.equal(c, again)
+        assert torch.equal(cb, c.to(torch.bfloat16))
+        assert torch.equal(acc, base + c)
+
+
+@pytest.mark.parametrize("B,S", [(1, 17), (1, 33), (2, 32), (1, 65), (5, 40), (1, 255)])
+def test_short_prompt_qkv(dev, B, S):
+    announce(f"short prompt qkv B={B} S={S}")
+    g = _gen(dev, S)
+    wqkv = bf16_randn(((HQ + 2 * HKV) * D, H), g, dev, std=0.02)
+    qn = (1.0 + 0.1 * torch.randn(D, generator=g, device=dev)).to(torch.bfloat16)
+    kn = (1.0 + 0.1 * torch.randn(D, generator=g, device=dev)).to(torch.bfloat16)
+    x = bf16_randn((B * S, H), g, dev)
+    pos = torch.arange(S, device=dev, dtype=torch.int32).repeat(B)
+    cos, sin = rope_tables(D, S, 1.0e6, dev)
+    kc = torch.zeros(B, HKV, S + 3, D, dtype=torch.bfloat16, device=dev)
+    vc = torch.zeros_like(kc)
+    q = ops.qkv_norm_rope(x, wqkv, qn, kn, cos, sin, pos, B, S, HQ, HKV, kc, vc, 1e-6)
+    torch.cuda.synchronize()
+    wq, wk, wv = wqkv.float().cpu().split([HQ * D, HKV * D, HKV * D])
+    rq, rk, rv = oracle.qkv_norm_rope(x.cpu().view(B, S, H), wq, wk, wv, qn.cpu(), kn.cpu(),
+                                      pos.cpu().view(B, S).long(), HQ, HKV, D, 1e-6, 1.0e6)
+    for a, r, what in ((q.view(B, S, HQ, D).transpose(1, 2), rq, "q"), (kc[:, :, :S], rk, "k"), (vc[:, :, :S], rv, "v")):
+        err = (a.float().cpu() - r).abs() - r.abs() * 2 ** -8  # one bf16 rounding
+        assert float(err.max()) <= 2e-4, what
+    assert int(kc[:, :, S:].abs().sum()) == 0
+
+
+@pytest.mark.parametrize("B", [9, 17, 40, 64, 65])
+def test_batched_decode_layer(dev, B):
+    """The attention layer's decode step, on both sides of the fused path's
+    limit, at ragged positions (one of them 0) against the same rows run as
+    batches of 8."""
+    announce(f"batched decode layer B={B}")
+    g = _gen(dev, B)
+    cap = 700
+    wqkv = bf16_randn(((HQ + 2 * HKV) * D, H), g, dev, std=0.02)
+    wo = bf16_randn((H, HQ * D), g, dev, std=0.02)
+    qn = (1.0 + 0.1 * torch.randn(D, generator=g, device=dev)).to(torch.bfloat16)
+    kn = (1.0 + 0.1 * torch.randn(D, generator=g, device=dev)).to(torch.bfloat16)
+    cos, sin = rope_tables(D, cap, 1.0e6, dev)
+    attn = Attention(wqkv, qn, kn, wo, HQ, HKV, D, 1e-6)
+    x = bf16_randn((B, H), g, dev)
+    pos = torch.randint(0, cap, (B,), generator=g, device=dev, dtype=torch.int32)
+    pos[0] = 0
+    cache = KVCache(B, HKV, cap, D, dev)
+    cache.k.normal_(0.0, 1.0, generator=g)
+    cache.v.normal_(0.0, 1.0, generator=g)
+    rows = torch.arange(B, device=dev)
+    k0, v0 = cache.k.clone(), cache.v.clone()
+    res = torch.randn(B, H, generator=g, device=dev)
+    out = attn.forward(x, res.clone(), pos, B, 1, cache, cos, sin)
+    for b0 in range(0, B, 8):
+        b1 = min(B, b0 + 8)
+        part = KVCache.wrap((k0[b0:b1].contiguous(), v0[b0:b1].contiguous()))
+        ref = attn.forward(x[b0:b1].contiguous(), res[b0:b1].clone(), pos[b0:b1].contiguous(), b1 - b0, 1, part, cos, sin)
+        torch.cuda.synchronize()
+        # bf16 q/k/v and attention output: one ulp apart where sums differ in order
+        assert_close_layer(out[b0:b1], ref, f"rows {b0}..{b1}", max_abs_tol=1e-2, mean_rel_tol=1e-3)
+        r = rows[b0:b1] - b0
+        for a, e in ((cache.k[b0:b1], part.k), (cache.v[b0:b1], part.v)):
+            new, want = a[r, :, pos[b0:b1].long()].float(), e[r, :, pos[b0:b1].long()].float()
+            # one bf16 step of the value, and the fp32 sums' order below it
+            assert bool(((new - want).abs() <= want.abs() * 2.0 ** -7 + 1e-5).all())
+            a[r, :, pos[b0:b1].long()] = e[r, :, pos[b0:b1].long()]
+            assert torch.equal(a, e)
