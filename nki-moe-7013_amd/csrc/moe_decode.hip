@@ -10,40 +10,42 @@
 // Grid: (active-expert slot, row group); slots beyond the number of touched
 // experts (meta[1]) exit at once, so the host sizes the grid as min(E, T*k)
 // without knowing the routing.  (The T <= 8 fused block is moe_block_decode.hip.)
-//
-// The token loop keeps the weight registers opaque to the optimiser: without
-// that, the loop-invariant bf16 -> fp32 unpacking is hoisted out of the loop,
-// doubling the live registers, and the weight loads get serialised.
 #include "decode_util.hpp"
+#include "mfma_pipe.hpp"
 
 namespace qmoe {
 
-// Token rows of gate/up staged in LDS at a time: small enough that several
-// workgroups share a CU, so each new workgroup's dependent first loads
-// (routing metadata, then its expert's rows) overlap the others' weight
-// streams.  4 rows (16 KB at H = 2048) leave room for five workgroups per
-// CU; 16 rows (64 KB) allowed two and made the gate/up pass 1.4x slower at
-// T = 64.
-#ifndef QMOE_GU_TOK_CHUNK
-#define QMOE_GU_TOK_CHUNK 4
-#endif
-constexpr int GU_TOK_CHUNK = QMOE_GU_TOK_CHUNK;
-
 // ================================================================== gate/up
 // Workgroup: 8 intermediate units (i0 = 8*blockIdx.y); wave w: units i0+2w,
-// i0+2w+1 = 2 gate rows + the 2 matching up rows of the packed w13.
-template <int HC, int TC>
+// i0+2w+1 = 2 gate rows + the 2 matching up rows of the packed w13, all in
+// registers (whole 1 KB row pieces per load, requested at once).  The
+// expert's tokens pass over them GU_TOK_CHUNK at a time: wave w copies token
+// c0 + w by LDS-DMA, the next chunk's copy in flight behind this chunk's dots
+// (v_dot2 on packed bf16 pairs, a wave reduction per row).  Bound by HBM
+// where experts hold a few tokens (16 tokens, 83 experts: 86 us for 522 MB).
+// A crowded expert's chunks used to wait for one copy after another: 32
+// tokens with 93 experts touched, 18 tokens in the largest, took 162 us for
+// 585 MB; 48 tokens with 46 in the largest 300 us.
+// Two chunks of 4 tokens (32 KB at H = 2048) leave room for five workgroups
+// per CU, so each new workgroup's dependent first loads (routing metadata,
+// then its expert's rows) overlap the others' weight streams.
+// (The rows as MFMA operands straight from global memory ran 5.2 TB/s
+// whatever the tile: 16 rows x 64 bytes per load are half lines.)
+constexpr int GU_TOK_CHUNK = 4;
+
+template <int HC>
 __global__ __launch_bounds__(256) void moe_gateup_gemv_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ w13,
     const int32_t* __restrict__ offsets, const int32_t* __restrict__ slot_token,
-    const int32_t* __restrict__ active, const int32_t* __restrict__ meta, int H, int I,
+    const int32_t* __restrict__ active, const int32_t* __restrict__ meta, int T, int I,
     float* __restrict__ act) {
-  extern __shared__ __attribute__((aligned(16))) uint16_t xs[];  // [TC][H]
+  constexpr int H = HC * 512, TC = GU_TOK_CHUNK;
+  __shared__ __attribute__((aligned(1024))) uint16_t xs[2][TC][H];
   // both requested before the branch (active has E >= gridDim.x entries)
   const int n_active = meta[1], e = active[blockIdx.x];
   if (int(blockIdx.x) >= n_active) return;
-  const int s0 = offsets[e], s1 = offsets[e + 1];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
   const int i_base = blockIdx.y * 8 + wave * 2;
   const int grp = i_base / 32, off = i_base % 32;
   const uint16_t* we = w13 + int64_t(e) * 2 * I * H;
@@ -55,22 +57,33 @@ __global__ __launch_bounds__(256) void moe_gateup_gemv_kernel(
 #pragma unroll
     for (int c = 0; c < HC; ++c) w[r][c] = ld_stream(p + c * 512);
   }
-  for (int c0 = s0; c0 < s1; c0 += TC) {
+  const int s0 = offsets[e], s1 = offsets[e + 1];
+  const pipe::i32x4 rx = pipe::make_rsrc(x, uint32_t(T) * uint32_t(H) * 2u);
+  const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>(&xs[0][wave][0]));
+  int tok = slot_token[min(s0 + wave, s1 - 1)];  // this wave's token of the next chunk to copy
+  auto copy = [&](int c0, int buf) {
+    if (c0 + wave < s1) {  // wave-uniform
+#pragma unroll
+      for (int c = 0; c < HC; ++c)
+        pipe::dma16(lds0 + uint32_t(buf * TC * H * 2 + c * 1024), uint32_t(lane * 16),
+                    rx, uint32_t(tok) * uint32_t(H * 2) + uint32_t(c * 1024));
+    }
+    tok = slot_token[min(c0 + TC + wave, s1 - 1)];
+  };
+  copy(s0, 0);
+  int buf = 0;
+  for (int c0 = s0; c0 < s1; c0 += TC, buf ^= 1) {
     const int n = min(TC, s1 - c0);
-    __syncthreads();
-    stage_rows_bf16(xs, x, slot_token, c0, n, H);
-    __syncthreads();
+    pipe::wait_vm<0>();  // this wave's part of the chunk (and its weights) has landed
+    lds_barrier();       // everyone's; and the other buffer's readers are done
+    if (c0 + TC < s1) copy(c0 + TC, buf ^ 1);
     for (int j = 0; j < n; ++j) {
       float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
       for (int c = 0; c < HC; ++c) {
-        float xf[8];
-        unpack8(*reinterpret_cast<const u32x4*>(xs + j * H + c * 512 + lane * 8), xf);
+        const u32x4 xv = *reinterpret_cast<const u32x4*>(&xs[buf][j][c * 512 + lane * 8]);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          opaque(w[r][c]);
-          acc[r] += dot8(w[r][c], xf);
-        }
+        for (int r = 0; r < 4; ++r) acc[r] = dot8_bf16(w[r][c], xv, acc[r]);
       }
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[r] = wave_sum(acc[r]);
@@ -202,14 +215,12 @@ static int launch_experts(const uint16_t* x, const uint16_t* w13, const uint16_t
                           const int32_t* meta, int64_t T, int64_t H, int64_t I, int64_t E, int64_t k,
                           float* act, float* y_slot, hipStream_t s) {
   const unsigned nact = unsigned(std::min<int64_t>(E, T * k));
-  // rows of one expert <= T*k (a token may list an expert twice via the seams)
-  const size_t shm1 = size_t(std::min<int64_t>(T * k, GU_TOK_CHUNK)) * H * 2;
   dim3 g1(nact, unsigned(I / 8));
   switch (H / 512) {
 #define QMOE_GU(HC)                                                                                  \
   case HC:                                                                                           \
-    hipLaunchKernelGGL((moe_gateup_gemv_kernel<HC, GU_TOK_CHUNK>), g1, dim3(256), shm1, s, x, w13,   \
-                       offsets, slot_token, active, meta, int(H), int(I), act);                     \
+    hipLaunchKernelGGL(moe_gateup_gemv_kernel<HC>, g1, dim3(256), 0, s, x, w13, offsets, slot_token, \
+                       active, meta, int(T), int(I), act);                                           \
     break;
     QMOE_GU(1)
     QMOE_GU(2)
