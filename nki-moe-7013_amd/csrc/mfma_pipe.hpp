@@ -61,6 +61,17 @@ __device__ __forceinline__ void dma16(uint32_t lds_addr, uint32_t voff, i32x4 rs
       : "memory");
 }
 
+// dma16 of bytes that are read once (non-temporal).
+__device__ __forceinline__ void dma16_nt(uint32_t lds_addr, uint32_t voff, i32x4 rsrc, uint32_t soff) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0\n\t"
+      "buffer_load_dwordx4 %1, %2, %3 offen nt lds"
+      :
+      : "s"(lds_addr), "v"(voff), "s"(rsrc), "s"(soff)
+      : "memory");
+}
+
 template <int N>
 __device__ __forceinline__ void wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");

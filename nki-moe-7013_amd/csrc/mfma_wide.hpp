@@ -44,7 +44,7 @@
 namespace qmoe {
 namespace pipe {
 
-template <int WA_, int FM_, int BK_, int S_, int BN_>
+template <int WA_, int FM_, int BK_, int S_, int BN_, bool NT_A = false>
 struct Wide {
   static constexpr int WA = WA_, FM = FM_;  // waves along A; A blocks per wave
   static constexpr int BM = 32 * FM * WA, BN = BN_, BK = BK_, S = S_, WAVES = 2 * WA, THREADS = 64 * WAVES;
@@ -98,7 +98,9 @@ struct Wide {
       const uint32_t soff_a = uint32_t(kt) * a_step, soff_b = uint32_t(kt) * b_step;
 #pragma unroll
       for (int j = part * NDMA / KS; j < (part + 1) * NDMA / KS; ++j) {
-        if (j < AI)
+        if (j < AI && NT_A)
+          dma16_nt(sb + uint32_t((wave * AI + j) * 1024), vo[j], ra, soff_a);
+        else if (j < AI)
           dma16(sb + uint32_t((wave * AI + j) * 1024), vo[j], ra, soff_a);
         else
           dma16(sb + uint32_t(A_BYTES + (wave * BI + (j - AI)) * 1024), vo[j], rb, soff_b);

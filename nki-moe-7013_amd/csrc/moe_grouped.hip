@@ -4,9 +4,11 @@
 // expert, runs of at most 256 expert-sorted slots.  Each item of work is one
 // (row tile, 256-row weight panel) pair on the direct-to-LDS pipeline of
 // mfma_wide.hpp (512 threads; A = 256 weight rows, B = up to 256 tokens; one
-// workgroup per CU).  Two pipelines share the kernel, chosen per tile:
-//   - more than 64 live rows: 256 x 256 x 32 stages, four deep, only the
+// workgroup per CU).  Three pipelines share the kernel, chosen per tile:
+//   - more than 128 live rows: 256 x 256 x 32 stages, four deep, only the
 //     live 32-row token blocks computed;
+//   - 65 to 128 live rows: 256 x 128 x 64 stages, three deep (2048 tokens over
+//     128 equally popular experts: 318 -> 296 us against the first one);
 //   - at most 64 live rows (cold experts, where streaming the weights is the
 //     whole cost): 256 x 64 x 64 stages, four deep, so three 32 KB weight
 //     slabs are in flight and one barrier covers 64 columns of K.
@@ -35,7 +37,7 @@
 namespace qmoe {
 
 namespace {
-// Full and partial tiles (more than 64 live rows): 256 x 256 x 32, four
+// Full and partial tiles (more than 128 live rows): 256 x 256 x 32, four
 // stages (three 32 KB stages in flight: a tile's weights are usually
 // streamed from HBM), 8 waves (2 per SIMD) of 64 x 128.
 using Hot = pipe::Wide<4, 2, 32, 4, 256>;
@@ -43,7 +45,11 @@ using Hot = pipe::Wide<4, 2, 32, 4, 256>;
 // four stages, so three 32 KB weight slabs are in flight and a barrier covers
 // 64 columns of K.
 using Cold = pipe::Wide<4, 2, 64, 4, 64>;
-constexpr int COLD_MAX_ROWS = Cold::BN;
+using ColdNt = pipe::Wide<4, 2, 64, 4, 64, true>;
+// 65 to 128 live rows: 256 x 128 x 64, three stages.
+using Warm = pipe::Wide<4, 2, 64, 3, 128>;
+using WarmNt = pipe::Wide<4, 2, 64, 3, 128, true>;
+constexpr int COLD_MAX_ROWS = Cold::BN, WARM_MAX_ROWS = Warm::BN;
 constexpr int PIPE_SMEM = Hot::SMEM > Cold::SMEM ? Hot::SMEM : Cold::SMEM;
 constexpr int PANEL = Hot::BM;
 static_assert(Hot::BM == Cold::BM && Hot::THREADS == Cold::THREADS, "one grid for both pipelines");
@@ -59,6 +65,7 @@ static_assert(SMEM <= 160 * 1024, "LDS");
 
 struct TileJob {
   int e, s0, rows, n0;
+  bool only;  // the expert's only tile: its weights are read once
 };
 
 // Work queues.  One persistent workgroup per CU takes (tile, weight panel)
@@ -151,13 +158,15 @@ __device__ __forceinline__ void finish_queue(int32_t* ctr, int32_t* done) {
   }
 }
 
-__device__ __forceinline__ TileJob job_of(int item, const int32_t* __restrict__ tiles, int npanels) {
+__device__ __forceinline__ TileJob job_of(int item, const int32_t* __restrict__ tiles, int n_tiles, int npanels) {
   TileJob job;
   const int t = item / npanels;
   job.n0 = (item - t * npanels) * PANEL;
   job.e = tiles[4 * t];
   job.s0 = tiles[4 * t + 1];
   job.rows = min(tiles[4 * t + 2] - job.s0, Hot::BN);
+  const int before = tiles[4 * max(t - 1, 0)], after = tiles[4 * min(t + 1, n_tiles - 1)];
+  job.only = (t == 0 || before != job.e) && (t == n_tiles - 1 || after != job.e);
   return job;
 }
 
@@ -282,6 +291,46 @@ __device__ __forceinline__ void down_tile(const TileJob& job, const uint16_t* ac
     *reinterpret_cast<uint4*>(dst + int64_t(r) * H + k * 8) = *reinterpret_cast<const uint4*>(tl + r * Y_LD + k * 8);
   }
 }
+
+// The pipeline of a tile, by its live rows and by whether its weights are
+// read once: a single-tile expert's weights are non-temporal on the pipelines
+// whose stages are whole 128-byte lines of a weight row (64 columns), which
+// streams them faster (300 tokens, 128 experts: 237 -> 215 us; 640: 246 ->
+// 229).  With several tiles the later ones find the panel in L2, and a
+// non-temporal read of it by the remainder tile cost the full tiles theirs
+// (4096 tokens over 128 equally popular experts: 440 -> 470 us), as did
+// non-temporal half lines on the 32-column stages.
+template <bool DEVICE>
+__device__ __forceinline__ void gateup_item(const TileJob& job, const uint16_t* __restrict__ x,
+                                            const uint16_t* __restrict__ w13, const int32_t* __restrict__ slot_token,
+                                            int T, int H, int I, uint16_t* act, uint8_t* smem) {
+  if (job.rows > WARM_MAX_ROWS)
+    gateup_tile<Hot, DEVICE>(job, x, w13, slot_token, T, H, I, act, smem);
+  else if (job.rows > COLD_MAX_ROWS)
+    if (job.only)
+      gateup_tile<WarmNt, DEVICE>(job, x, w13, slot_token, T, H, I, act, smem);
+    else
+      gateup_tile<Warm, DEVICE>(job, x, w13, slot_token, T, H, I, act, smem);
+  else if (job.only)
+    gateup_tile<ColdNt, DEVICE>(job, x, w13, slot_token, T, H, I, act, smem);
+  else
+    gateup_tile<Cold, DEVICE>(job, x, w13, slot_token, T, H, I, act, smem);
+}
+
+__device__ __forceinline__ void down_item(const TileJob& job, const uint16_t* act, const uint16_t* __restrict__ w2,
+                                          int slots, int H, int I, uint16_t* __restrict__ y_slot, uint8_t* smem) {
+  if (job.rows > WARM_MAX_ROWS || I % Cold::BK != 0)
+    down_tile<Hot>(job, act, w2, slots, H, I, y_slot, smem);
+  else if (job.rows > COLD_MAX_ROWS)
+    if (job.only)
+      down_tile<WarmNt>(job, act, w2, slots, H, I, y_slot, smem);
+    else
+      down_tile<Warm>(job, act, w2, slots, H, I, y_slot, smem);
+  else if (job.only)
+    down_tile<ColdNt>(job, act, w2, slots, H, I, y_slot, smem);
+  else
+    down_tile<Cold>(job, act, w2, slots, H, I, y_slot, smem);
+}
 }  // namespace
 
 __global__ __launch_bounds__(Hot::THREADS, 1) void moe_gateup_grouped_kernel(
@@ -293,12 +342,9 @@ __global__ __launch_bounds__(Hot::THREADS, 1) void moe_gateup_grouped_kernel(
   int32_t* ctr = meta + META_CTR;
   const Queue qu(ctr, live, xcd);
   for (int item = next_item(qu, NO_RESERVE, smem); item >= 0;) {
-    const TileJob job = job_of(item, tiles, npanels);
+    const TileJob job = job_of(item, tiles, meta[0], npanels);
     const int reserve = job.rows <= COLD_MAX_ROWS ? reserve_own(qu, item) : NO_RESERVE;
-    if (job.rows <= COLD_MAX_ROWS)
-      gateup_tile<Cold, false>(job, x, w13, slot_token, T, H, I, act, smem);
-    else
-      gateup_tile<Hot, false>(job, x, w13, slot_token, T, H, I, act, smem);
+    gateup_item<false>(job, x, w13, slot_token, T, H, I, act, smem);
     item = next_item(qu, reserve, smem);
   }
   finish_queue(ctr, meta + META_DONE);
@@ -313,12 +359,9 @@ __global__ __launch_bounds__(Hot::THREADS, 1) void moe_down_grouped_kernel(
   int32_t* ctr = meta + META_CTR + 8;
   const Queue qu(ctr, live, xcd);
   for (int item = next_item(qu, NO_RESERVE, smem); item >= 0;) {
-    const TileJob job = job_of(item, tiles, npanels);
+    const TileJob job = job_of(item, tiles, meta[0], npanels);
     const int reserve = job.rows <= COLD_MAX_ROWS ? reserve_own(qu, item) : NO_RESERVE;
-    if (job.rows <= COLD_MAX_ROWS && I % Cold::BK == 0)
-      down_tile<Cold>(job, act, w2, slots, H, I, y_slot, smem);
-    else
-      down_tile<Hot>(job, act, w2, slots, H, I, y_slot, smem);
+    down_item(job, act, w2, slots, H, I, y_slot, smem);
     item = next_item(qu, reserve, smem);
   }
   finish_queue(ctr, meta + META_DONE + 1);
@@ -363,12 +406,9 @@ __global__ __launch_bounds__(Hot::THREADS, 1) void moe_experts_fused_kernel(
   {
     const Queue qu(meta + META_CTR, n_tiles * np1, xcd);
     for (int item = next_item(qu, NO_RESERVE, smem); item >= 0;) {
-      const TileJob job = job_of(item, tiles, np1);
+      const TileJob job = job_of(item, tiles, n_tiles, np1);
       const int reserve = job.rows <= COLD_MAX_ROWS ? reserve_own(qu, item) : NO_RESERVE;
-      if (job.rows <= COLD_MAX_ROWS)
-        gateup_tile<Cold, true>(job, x, w13, slot_token, T, H, I, act, smem);
-      else
-        gateup_tile<Hot, true>(job, x, w13, slot_token, T, H, I, act, smem);
+      gateup_item<true>(job, x, w13, slot_token, T, H, I, act, smem);
       __syncthreads();  // every wave's act stores are complete
       if (threadIdx.x == 0)
         __hip_atomic_fetch_add(tiles + 4 * (item / np1) + 3, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -378,13 +418,10 @@ __global__ __launch_bounds__(Hot::THREADS, 1) void moe_experts_fused_kernel(
   {
     const Queue qu(meta + META_CTR + 8, n_tiles * np2, xcd);
     for (int item = next_item(qu, NO_RESERVE, smem); item >= 0;) {
-      const TileJob job = job_of(item, tiles, np2);
+      const TileJob job = job_of(item, tiles, n_tiles, np2);
       wait_tile(tiles + 4 * (item / np2) + 3, np1, meta);
       const int reserve = job.rows <= COLD_MAX_ROWS ? reserve_own(qu, item) : NO_RESERVE;
-      if (job.rows <= COLD_MAX_ROWS && I % Cold::BK == 0)
-        down_tile<Cold>(job, act, w2, slots, H, I, y_slot, smem);
-      else
-        down_tile<Hot>(job, act, w2, slots, H, I, y_slot, smem);
+      down_item(job, act, w2, slots, H, I, y_slot, smem);
       item = next_item(qu, reserve, smem);
     }
   }
