@@ -418,6 +418,106 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(const uint16_t*
   }
 }
 
+// Vocabulary-size projections of 2 <= M <= 64 rows (batched lm_head): N
+// columns in tiles of 16, persistent workgroups taking every gridDim-th tile.
+// Wave w of the K / 256 owns k in [256 w, 256 w + 256): its A fragments stay
+// in registers for the whole launch (re-reading them per workgroup is what
+// the column-owning kernels above spend their time on here), and its slice of
+// a tile's weight rows (16 x 512 bytes: whole lines, non-temporal) streams
+// through a private LDS ring of VO_S tiles without workgroup barriers.  The
+// waves' partial tiles are added in k order through LDS, one barrier a tile.
+// Bound by the weight stream: 622 MB (N = 151936, K = 2048).
+constexpr int VO_S = 2, VO_TILE = 16 * 512;
+// Row m of a partial tile sits at vo_row(m): the four lane groups' rows (4
+// apart) are neighbours, so their stores and the sums' reads hit all banks.
+__device__ __forceinline__ int vo_row(int m) { return (m & ~15) | ((m & 3) << 2) | ((m >> 2) & 3); }
+template <int WAVES, int MT>
+struct Vocab {
+  static constexpr int RED = WAVES * MT * 256 * 4;  // bytes of one set of partial tiles
+  static constexpr int NRED = WAVES * VO_S * VO_TILE + 2 * RED <= 160 * 1024 ? 2 : 1;
+  static constexpr int SMEM = WAVES * VO_S * VO_TILE + NRED * RED;
+};
+template <int WAVES, int MT, int MODE>
+__global__ __launch_bounds__(64 * WAVES) void gemm_vocab_kernel(const uint16_t* __restrict__ A, int64_t lda,
+                                                                const uint16_t* __restrict__ B, int M, int N,
+                                                                int K, void* __restrict__ C, int64_t ldc) {
+  using V = Vocab<WAVES, MT>;
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];  // rings, then partial tiles
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const int col = lane & 15, kg = lane >> 4, kw = wave * 256;
+  const int tiles = (N + 15) / 16;
+  uint8_t* ring = smem + wave * (VO_S * VO_TILE);
+  const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>(ring));
+  const pipe::i32x4 rb = pipe::make_rsrc(B, uint32_t(int64_t(N) * K * 2));
+  // DMA instruction i: rows 2i, 2i + 1 of the tile; chunk c of row r at slot c ^ r (32 chunks of 16 bytes a row)
+  uint32_t vo[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int r = 2 * i + (lane >> 5);
+    vo[i] = uint32_t(r) * uint32_t(K * 2) + uint32_t(kw * 2 + ((lane & 31) ^ r) * 16);
+  }
+  auto copy = [&](int tile, int slot) {
+    const uint32_t base = uint32_t(tile) * 16u * uint32_t(K * 2);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int r = 2 * i + (lane >> 5);
+      pipe::dma16_nt(lds0 + uint32_t(slot * VO_TILE + i * 1024), tile * 16 + r < N ? vo[i] + base : pipe::PAD, rb, 0);
+    }
+  };
+  bf16x8 af[MT][8];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {  // rows past M repeat the last one; their products are not stored
+    const uint16_t* p = A + int64_t(min(i * 16 + col, M - 1)) * lda + kw + kg * 8;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) af[i][s] = *reinterpret_cast<const bf16x8*>(p + s * 32);
+  }
+  int tile = blockIdx.x;
+#pragma unroll
+  for (int s = 0; s < VO_S; ++s)
+    if (tile + s * int(gridDim.x) < tiles) copy(tile + s * gridDim.x, s);
+  for (int it = 0; tile < tiles; tile += gridDim.x, ++it) {
+    const int slot = it % VO_S;
+    const bool more = tile + VO_S * int(gridDim.x) < tiles;
+    // the tile has landed when only the copies issued after it are pending
+    // (the stores in between make this wait for a little more than that)
+    if (tile + int(gridDim.x) < tiles)
+      pipe::wait_vm<8 * (VO_S - 1)>();
+    else
+      pipe::wait_vm<0>();
+    const uint8_t* wt = ring + slot * VO_TILE + col * 512;
+    bf16x8 bf[8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) bf[s] = *reinterpret_cast<const bf16x8*>(wt + ((s * 4 + kg) ^ col) * 16);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot is read: its next copy may land
+    if (more) copy(tile + VO_S * gridDim.x, slot);
+    f32x4 acc[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) acc[i] = f32x4{};
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+#pragma unroll
+      for (int i = 0; i < MT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i][s], bf[s], acc[i], 0, 0, 0);
+    // lane l holds column l % 16, rows 16 i + (l / 16) * 4 + 0..3
+    float* red = reinterpret_cast<float*>(smem + WAVES * VO_S * VO_TILE + (it % V::NRED) * V::RED);
+    if (V::NRED == 1) lds_barrier();  // the previous tile's sums are read
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) red[(wave * MT * 16 + i * 16 + e * 4 + kg) * 16 + col] = acc[i][e];
+    lds_barrier();
+    for (int i = threadIdx.x; i < MT * 256; i += 64 * WAVES) {
+      const int m = vo_row(i >> 4), n = i & 15;  // vo_row is its own inverse
+      if (m < M && tile * 16 + n < N) {
+        float v = red[i];
+#pragma unroll
+        for (int w = 1; w < WAVES; ++w) v += red[w * MT * 256 + i];
+        store_out<MODE>(C, int64_t(m) * ldc + tile * 16 + n, v);
+      }
+    }
+  }
+}
+
 // ------------------------------------------------------------------ MFMA tile
 // Grid = every (row tile, column tile) pair, renumbered XCD-contiguously and
 // then walked in groups of 8 row tiles per column sweep, so the workgroups
@@ -1108,11 +1208,55 @@ static int launch_gemv_pk(const uint16_t* A, int64_t lda, const uint16_t* B, int
 // before (16-row GEMV, 64 x 64 tiles), 9 / 16 / 32 / 64 rows: N = 5120, K =
 // 2048 8.9 / 11.5 / 12.1 / 13.0 -> 6.2 / 6.9 / 8.8 / 12.5 us; N = 2048, K =
 // 4096 20.5 / 20.8 / 21.8 / 23.1 -> 6.5 / 7.8 / 10.9 / 18.2 us.  At the
-// vocabulary's N = 151936 every one of 7597 workgroups re-reads A and the
-// tiles stay ahead (135 / 169 / 179 us against 148 / 222 / 314 at 12 / 32 / 64).
+// vocabulary's N = 151936 every one of 7597 workgroups re-reads A (148 / 222 /
+// 314 us at 12 / 32 / 64 rows): gemm_vocab_kernel's.
 static bool skinny_ok(int64_t M, int64_t N, int64_t K) {
   return M >= 9 && M <= 64 && (K == 512 || K == 1024 || K == 2048 || K == 4096) && N * K * 2 < (1ll << 31) &&
          N <= 40ll * current_device_cus();
+}
+
+// Rows and shapes of gemm_vocab_kernel: the column counts above the skinny
+// kernel's.  N = 151936, K = 2048 at 2 / 8 / 16 / 32 / 64 rows, against the
+// packed GEMV, the 16-row GEMV and the 256 x 256 tiles: 118 / 131 / 149 / 159 /
+// 169 -> 102 / 109 / 116 / 122 / 132 us (6.1 to 4.7 TB/s, of which the fp32
+// output takes 1 to 39 MB); N = 20000, K = 1024, 32 rows 19.4 -> 11.6 us.  At K = 512 a
+// tile is too short for its barrier (N = 10243, 33 rows: 5.1 -> 6.8 us).
+static bool vocab_ok(int64_t M, int64_t N, int64_t K) {
+  return M >= 2 && M <= 64 && (K == 1024 || K == 2048) && N * K * 2 < (1ll << 31) &&
+         N > 40ll * current_device_cus();
+}
+
+template <int WAVES, int MT, int MODE>
+static int launch_vocab_t(const uint16_t* A, int64_t lda, const uint16_t* B, int M, int N, int K, void* C,
+                          int64_t ldc, hipStream_t s) {
+  constexpr int SMEM = Vocab<WAVES, MT>::SMEM;
+  static_assert(SMEM <= 160 * 1024, "LDS");
+  static const bool attr = [] {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_vocab_kernel<WAVES, MT, MODE>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, SMEM);
+    return true;
+  }();
+  (void)attr;
+  const int64_t groups = int64_t(std::max(current_device_cus(), 1)) * (8 / WAVES);
+  hipLaunchKernelGGL((gemm_vocab_kernel<WAVES, MT, MODE>), dim3(unsigned(std::min<int64_t>((N + 15) / 16, groups))),
+                     dim3(64 * WAVES), SMEM, s, A, lda, B, M, N, K, C, ldc);
+  return hip_status("qmoe_gemm(vocab)");
+}
+
+template <int WAVES, int MODE>
+static int launch_vocab_w(const uint16_t* A, int64_t lda, const uint16_t* B, int M, int N, int K, void* C,
+                          int64_t ldc, hipStream_t s) {
+  return M <= 16   ? launch_vocab_t<WAVES, 1, MODE>(A, lda, B, M, N, K, C, ldc, s)
+         : M <= 32 ? launch_vocab_t<WAVES, 2, MODE>(A, lda, B, M, N, K, C, ldc, s)
+         : M <= 48 ? launch_vocab_t<WAVES, 3, MODE>(A, lda, B, M, N, K, C, ldc, s)
+                   : launch_vocab_t<WAVES, 4, MODE>(A, lda, B, M, N, K, C, ldc, s);
+}
+
+template <int MODE>
+static int launch_vocab(const uint16_t* A, int64_t lda, const uint16_t* B, int M, int N, int K, void* C,
+                        int64_t ldc, hipStream_t s) {
+  return K == 1024 ? launch_vocab_w<4, MODE>(A, lda, B, M, N, K, C, ldc, s)
+                   : launch_vocab_w<8, MODE>(A, lda, B, M, N, K, C, ldc, s);
 }
 
 template <int WAVES, int NB, int MT, int MODE>
@@ -1206,6 +1350,16 @@ int gemm_launch(const uint16_t* A, int64_t lda, const uint16_t* B, int64_t M, in
   QMOE_REQUIRE(lda % 8 == 0, "qmoe_gemm: lda must be a multiple of 8");
   QMOE_REQUIRE(M < (1ll << 31) && N < (1ll << 31) && K < (1ll << 31), "qmoe_gemm: dims overflow");
   if (M == 0) return QMOE_OK;
+  if (vocab_ok(M, N, K)) {
+    switch (mode) {
+      case QMOE_GEMM_STORE_BF16:
+        return launch_vocab<QMOE_GEMM_STORE_BF16>(A, lda, B, int(M), int(N), int(K), C, ldc, s);
+      case QMOE_GEMM_STORE_F32:
+        return launch_vocab<QMOE_GEMM_STORE_F32>(A, lda, B, int(M), int(N), int(K), C, ldc, s);
+      default:
+        return launch_vocab<QMOE_GEMM_ADD_F32>(A, lda, B, int(M), int(N), int(K), C, ldc, s);
+    }
+  }
   if (skinny_ok(M, N, K) && (M - 1) * lda * 2 + K * 2 < (1ll << 31)) {
     switch (mode) {
       case QMOE_GEMM_STORE_BF16:

@@ -52,26 +52,38 @@ __device__ __forceinline__ uint64_t block_max_u64(uint64_t k, uint64_t* red) {
   return m;
 }
 
+// Workgroup (slice p of gridDim.x, row): AM_U values per thread in flight.
+// Many rows take fewer, longer slices (argmax_parts): with 256 slices a row,
+// 32 rows of 151,936 were 8192 workgroups of two loads a thread, one after
+// the other: 13 us for 19 MB.
+constexpr int AM_U = 8;
 __global__ __launch_bounds__(ARGMAX_THREADS) void argmax_partial_kernel(const float* __restrict__ x,
                                                                         int64_t n, int64_t ldx,
                                                                         uint64_t* __restrict__ part) {
   __shared__ uint64_t red[ARGMAX_THREADS / 64];
   const int row = blockIdx.y, p = blockIdx.x;
-  const int64_t chunk = (n + ARGMAX_PARTS - 1) / ARGMAX_PARTS;
+  const int64_t chunk = (n + gridDim.x - 1) / gridDim.x;
   const int64_t b0 = int64_t(p) * chunk, b1 = min(n, b0 + chunk);
   const float* xr = x + int64_t(row) * ldx;
   uint64_t k = 0;  // below every real key (index complement of -1 never wins)
-  for (int64_t i = b0 + threadIdx.x; i < b1; i += ARGMAX_THREADS) k = u64max(k, argmax_key(xr[i], i));
+  for (int64_t i = b0 + threadIdx.x; i < b1; i += ARGMAX_THREADS * AM_U) {
+    float v[AM_U];
+#pragma unroll
+    for (int u = 0; u < AM_U; ++u) v[u] = xr[min(i + u * ARGMAX_THREADS, b1 - 1)];
+#pragma unroll
+    for (int u = 0; u < AM_U; ++u)  // a value past the slice is its last one again: the same key
+      k = u64max(k, argmax_key(v[u], min(i + u * ARGMAX_THREADS, b1 - 1)));
+  }
   k = block_max_u64(k, red);
   if (threadIdx.x == 0) part[int64_t(row) * ARGMAX_PARTS + p] = k;
 }
 
 __global__ __launch_bounds__(ARGMAX_THREADS) void argmax_final_kernel(const uint64_t* __restrict__ part,
-                                                                      int64_t* __restrict__ out) {
+                                                                      int parts, int64_t* __restrict__ out) {
   __shared__ uint64_t red[ARGMAX_THREADS / 64];
   const int row = blockIdx.x;
   uint64_t k = 0;
-  for (int i = threadIdx.x; i < ARGMAX_PARTS; i += ARGMAX_THREADS)
+  for (int i = threadIdx.x; i < parts; i += ARGMAX_THREADS)
     k = u64max(k, part[int64_t(row) * ARGMAX_PARTS + i]);
   k = block_max_u64(k, red);
   if (threadIdx.x == 0) out[row] = int64_t(~uint32_t(k & 0xffffffffu));
@@ -112,10 +124,12 @@ extern "C" int qmoe_argmax(const float* x, int64_t rows, int64_t n, int64_t ldx,
   if (rows == 0) return QMOE_OK;
   hipStream_t s = as_stream(stream);
   uint64_t* part = static_cast<uint64_t*>(workspace);
-  hipLaunchKernelGGL(argmax_partial_kernel, dim3(ARGMAX_PARTS, unsigned(rows)), dim3(ARGMAX_THREADS), 0,
+  // slices of a row: all 256 for a few rows, then about 1024 workgroups, at least 8 a row
+  const int parts = int(std::min<int64_t>(ARGMAX_PARTS, std::max<int64_t>(8, 1024 / rows)));
+  hipLaunchKernelGGL(argmax_partial_kernel, dim3(parts, unsigned(rows)), dim3(ARGMAX_THREADS), 0,
                      s, x, n, ldx, part);
   if (int rc = hip_status("qmoe_argmax(partial)")) return rc;
-  hipLaunchKernelGGL(argmax_final_kernel, dim3(unsigned(rows)), dim3(ARGMAX_THREADS), 0, s, part, out);
+  hipLaunchKernelGGL(argmax_final_kernel, dim3(unsigned(rows)), dim3(ARGMAX_THREADS), 0, s, part, parts, out);
   return hip_status("qmoe_argmax(final)");
 }
 

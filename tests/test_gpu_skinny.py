@@ -30,7 +30,7 @@ def test_skinny_gemm(dev, M, N, K):
     base = torch.randn(M, N, generator=g, device=dev)
     ref = A.double() @ B.double().t()
     # fp32 sums of K products in any order: K * 2^-24 of the sum of magnitudes
-    bound = (A.double().abs() @ B.double().abs().t()) * (K * 2.0 ** -24)
+    bound = (A.double().abs() @ B.double().abs().t()).mul_(K * 2.0 ** -24)
     ws = ops.gemm_workspace(M, N, K, dev)
     for w in (None, ws) if ws is not None else (None,):
         c = ops.gemm(A, B, _lib.GEMM_STORE_F32, workspace=w)
@@ -43,6 +43,33 @@ def test_skinny_gemm(dev, M, N, K):
         assert torch.equal(c, again)
         assert torch.equal(cb, c.to(torch.bfloat16))
         assert torch.equal(acc, base + c)
+
+
+# the vocabulary kernel: row-tile edges, a last tile of one column, fewer and
+# more tiles than a round of workgroups, both K
+@pytest.mark.parametrize("M", [2, 8, 9, 16, 17, 33, 48, 64])
+@pytest.mark.parametrize("N,K", [(10241, 2048), (12289, 1024), (40001, 2048)])
+def test_vocab_gemm(dev, M, N, K):
+    test_skinny_gemm(dev, M, N, K)
+
+
+# every slice count of the partial pass (256, 34, 8), slices longer and shorter
+# than a thread's eight values, rows of one value
+@pytest.mark.parametrize("rows,n", [(1, 1), (3, 255), (4, 151936), (30, 20011), (64, 151936), (130, 4097), (300, 7)])
+def test_argmax_slices(dev, rows, n):
+    announce(f"argmax rows={rows} n={n}")
+    g = _gen(dev, rows + n)
+    x = torch.randn(rows, n, generator=g, device=dev)
+    x[0] = float("-inf")
+    if rows > 1:
+        x[1, :] = 1.5  # all equal: the first wins
+    if rows > 2:
+        x[2, n - 1] = float("inf")
+    got = ops.argmax(x)
+    torch.cuda.synchronize()
+    best = x.cpu().max(dim=1).values.unsqueeze(1)
+    first = (x.cpu() == best).float().argmax(dim=1)
+    assert torch.equal(got.cpu(), first)
 
 
 @pytest.mark.parametrize("B,S", [(1, 17), (1, 33), (2, 32), (1, 65), (5, 40), (1, 255)])
