@@ -7,9 +7,12 @@
 //   moe_down_mfma_kernel     y_slot[s,h] = bf16(act[s]).W2[e,h] (fp32 accumulation)
 //                            on MFMA, from the blocked w2 layout [E][I/8][H][8].
 //
-// Grid: (active-expert slot, row group); slots beyond the number of touched
+// Grid: (row group, active-expert slot); slots beyond the number of touched
 // experts (meta[1]) exit at once, so the host sizes the grid as min(E, T*k)
-// without knowing the routing.  (The T <= 8 fused block is moe_block_decode.hip.)
+// without knowing the routing.  Row groups are the fastest index: an expert's
+// workgroups then go round the 8 XCDs (with 128 slots fastest, each expert
+// had its XCD and a crowded one kept it busy alone: 48 tokens, 46 of them in
+// one expert, 237 -> 139 us; equally popular experts 177 -> 172 us at 32).  (The T <= 8 fused block is moe_block_decode.hip.)
 #include "decode_util.hpp"
 #include "mfma_pipe.hpp"
 
@@ -42,11 +45,11 @@ __global__ __launch_bounds__(256) void moe_gateup_gemv_kernel(
   constexpr int H = HC * 512, TC = GU_TOK_CHUNK;
   __shared__ __attribute__((aligned(1024))) uint16_t xs[2][TC][H];
   // both requested before the branch (active has E >= gridDim.x entries)
-  const int n_active = meta[1], e = active[blockIdx.x];
-  if (int(blockIdx.x) >= n_active) return;
+  const int n_active = meta[1], e = active[blockIdx.y];
+  if (int(blockIdx.y) >= n_active) return;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
-  const int i_base = blockIdx.y * 8 + wave * 2;
+  const int i_base = blockIdx.x * 8 + wave * 2;
   const int grp = i_base / 32, off = i_base % 32;
   const uint16_t* we = w13 + int64_t(e) * 2 * I * H;
   u32x4 w[4][HC];  // rows: gate i_base, gate i_base+1, up i_base, up i_base+1
@@ -120,10 +123,10 @@ __global__ __launch_bounds__(256) void moe_down_mfma_kernel(
     const int32_t* __restrict__ offsets, const int32_t* __restrict__ active,
     const int32_t* __restrict__ meta, int H, int I, float* __restrict__ y_slot) {
   extern __shared__ __attribute__((aligned(16))) uint16_t as[];  // hi, lo: [2][DN_ROWS][I + 8] bf16
-  const int n_active = meta[1], e = active[blockIdx.x];  // both requested before the branch
-  if (int(blockIdx.x) >= n_active) return;
+  const int n_active = meta[1], e = active[blockIdx.y];  // both requested before the branch
+  if (int(blockIdx.y) >= n_active) return;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6, col = lane & 15, kq = lane >> 4;
-  const int h = blockIdx.y * DN_COLS + wave * 16 + col;
+  const int h = blockIdx.x * DN_COLS + wave * 16 + col;
   const int NS = I / QMOE_W2_BLOCK, KS = I / 32, ald = I + 8;
   const int nkb = (KS + DN_KB - 1) / DN_KB;
   // block kb = 4*ks + kq of column h: w2b[((e*NS + kb)*H + h)*8 .. +8]
@@ -215,7 +218,7 @@ static int launch_experts(const uint16_t* x, const uint16_t* w13, const uint16_t
                           const int32_t* meta, int64_t T, int64_t H, int64_t I, int64_t E, int64_t k,
                           float* act, float* y_slot, hipStream_t s) {
   const unsigned nact = unsigned(std::min<int64_t>(E, T * k));
-  dim3 g1(nact, unsigned(I / 8));
+  dim3 g1(unsigned(I / 8), nact);
   switch (H / 512) {
 #define QMOE_GU(HC)                                                                                  \
   case HC:                                                                                           \
@@ -231,7 +234,7 @@ static int launch_experts(const uint16_t* x, const uint16_t* w13, const uint16_t
   int rc = hip_status("moe experts (gate_up)");
   if (rc) return rc;
   const size_t shm2 = size_t(2 * DN_ROWS) * (I + 8) * 2;
-  dim3 g2(nact, unsigned(H / DN_COLS));
+  dim3 g2(unsigned(H / DN_COLS), nact);
   hipLaunchKernelGGL(moe_down_mfma_kernel, g2, dim3(256), shm2, s, act, w2, offsets, active, meta, int(H),
                      int(I), y_slot);
   return hip_status("moe experts (down)");
