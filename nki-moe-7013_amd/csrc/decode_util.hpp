@@ -37,17 +37,4 @@ __device__ __forceinline__ void stage16(u32x4* dst, int n, Src src) {
   for (int c = int(threadIdx.x) + NT * MAXI; c < n; c += NT) dst[c] = ld16(src(c));
 }
 
-// Stage n token rows (bf16 [H]) into LDS; rows given by an index map or direct.
-// A plain strided loop: it keeps the caller's registers free, which matters
-// more than batching these loads where several workgroups share a CU.
-__device__ __forceinline__ void stage_rows_bf16(uint16_t* dst, const uint16_t* src,
-                                                const int32_t* row_map, int r0, int n, int H) {
-  const int hch = H / 8;
-  for (int q = threadIdx.x; q < n * hch; q += blockDim.x) {
-    const int j = q / hch, kc = q - j * hch;
-    const int64_t row = row_map ? row_map[r0 + j] : (r0 + j);
-    *reinterpret_cast<u32x4*>(dst + j * H + kc * 8) = ld16(src + row * H + kc * 8);
-  }
-}
-
 }  // namespace qmoe

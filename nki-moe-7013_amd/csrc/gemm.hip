@@ -1,11 +1,15 @@
 // Dense bf16 GEMM  C = A . B^T  (A [M,K], B [N,K], fp32 accumulate).
 //
-// Two shapes of work:
-//  * M <= 16 ("GEMV", decode): HBM-bound on B.  The M activation rows are
+// Three shapes of work:
+//  * M <= 8 ("GEMV", decode; to 16 where the next kernels do not apply):
+//    HBM-bound on B.  The M activation rows are
 //    staged once in LDS; each wave streams R rows of B with 16-byte
 //    non-temporal loads (K/512 loads per row per lane, all in flight), and
 //    reduces the per-lane partial dots with cross-lane shuffles.
-//  * M > 16: the direct-to-LDS MFMA pipelines (mfma_pipe.hpp; from 224
+//  * 9 <= M <= 64 (batched decode, from 2 rows at vocabulary-size N): the
+//    weights stream through LDS past the rows (gemm_skinny_kernel,
+//    gemm_slice_kernel, gemm_vocab_kernel).
+//  * larger M: the direct-to-LDS MFMA pipelines (mfma_pipe.hpp; from 224
 //    tiles of 256 x 256 on, the deep-staged 8-wave one of mfma_wide.hpp).
 #include "decode_util.hpp"
 #include "gemm.hpp"

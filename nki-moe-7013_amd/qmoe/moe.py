@@ -23,9 +23,10 @@ import torch
 from . import _lib, ops
 
 # Token counts at or below this use the HBM-bound GEMV experts; above it the
-# MFMA grouped GEMM.  (Each touched expert is streamed once either way; with
-# 128 experts the two paths take the same time at T = 48 on MI355X: 242 us
-# per block, against 212 / 233 us at T = 32 and 270 / 248 us at T = 64.)
+# MFMA grouped GEMM.  (Each touched expert is streamed once either way.  With
+# 128 equally popular experts the GEMV form is ahead, 190 against 213 us at
+# T = 48 and 193 against 216 us at 64; where a few experts hold most tokens
+# the grouped one is, 116 against 136 us at 48 and 137 against 164 us at 64.)
 GEMV_MAX_TOKENS = 48
 # Row tile of the prefill dispatch table: one (up to) 256 x 256 MFMA tile per
 # (tile, panel).
