@@ -1273,8 +1273,10 @@ extern "C" int qmoe_qkv_norm_rope(const qmoe_bf16* x, const qmoe_bf16* wqkv,
                            max_p, eps, q_out, k_cache, v_cache, as_stream(stream));
   // The direct-to-LDS pipelines take every other row count (17 to 255 rows,
   // which the register-staged 128 x 128 tiles ran in 55-60 us, take 17-20 us on
-  // the 64-row tiles); the register-staged kernel keeps x of 4 GiB and more.
-  if (T * H * 2 < (1ll << 32)) {
+  // the 64-row tiles); the register-staged kernel keeps x of 4 GiB and more,
+  // and below 256 rows operands that are not 16-byte aligned.
+  const bool aligned = (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(wqkv)) % 16 == 0;
+  if (T * H * 2 < (1ll << 32) && (aligned || T >= 256)) {
     // 256-row tiles once they give every CU a workgroup; below that 128-row
     // tiles, two per CU, while they fill the CUs.  Fewer tiles than CUs: one
     // workgroup per CU with four stages in flight, 64-row tiles while those

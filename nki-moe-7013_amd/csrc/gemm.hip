@@ -1207,6 +1207,10 @@ static int launch_gemv_pk(const uint16_t* A, int64_t lda, const uint16_t* B, int
   return fail(QMOE_ERR_INVALID, "qmoe_gemm: packed GEMV needs K in {512, 1024, 2048, 4096}");
 }
 
+// B is copied by LDS-DMA, 16 bytes a lane: a B that is not 16-byte aligned
+// stays on the kernels that load it into registers.
+static bool dma_aligned(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
 // Rows and shapes that gemm_skinny_kernel takes: up to two rounds of its
 // 20-column workgroups.  Measured against the kernels that took these shapes
 // before (16-row GEMV, 64 x 64 tiles), 9 / 16 / 32 / 64 rows: N = 5120, K =
@@ -1214,8 +1218,8 @@ static int launch_gemv_pk(const uint16_t* A, int64_t lda, const uint16_t* B, int
 // 4096 20.5 / 20.8 / 21.8 / 23.1 -> 6.5 / 7.8 / 10.9 / 18.2 us.  At the
 // vocabulary's N = 151936 every one of 7597 workgroups re-reads A (148 / 222 /
 // 314 us at 12 / 32 / 64 rows): gemm_vocab_kernel's.
-static bool skinny_ok(int64_t M, int64_t N, int64_t K) {
-  return M >= 9 && M <= 64 && (K == 512 || K == 1024 || K == 2048 || K == 4096) && N * K * 2 < (1ll << 31) &&
+static bool skinny_ok(const void* B, int64_t M, int64_t N, int64_t K) {
+  return dma_aligned(B) && M >= 9 && M <= 64 && (K == 512 || K == 1024 || K == 2048 || K == 4096) && N * K * 2 < (1ll << 31) &&
          N <= 40ll * current_device_cus();
 }
 
@@ -1225,8 +1229,8 @@ static bool skinny_ok(int64_t M, int64_t N, int64_t K) {
 // 169 -> 102 / 109 / 116 / 122 / 132 us (6.1 to 4.7 TB/s, of which the fp32
 // output takes 1 to 39 MB); N = 20000, K = 1024, 32 rows 19.4 -> 11.6 us.  At K = 512 a
 // tile is too short for its barrier (N = 10243, 33 rows: 5.1 -> 6.8 us).
-static bool vocab_ok(int64_t M, int64_t N, int64_t K) {
-  return M >= 2 && M <= 64 && (K == 1024 || K == 2048) && N * K * 2 < (1ll << 31) &&
+static bool vocab_ok(const void* B, int64_t M, int64_t N, int64_t K) {
+  return dma_aligned(B) && M >= 2 && M <= 64 && (K == 1024 || K == 2048) && N * K * 2 < (1ll << 31) &&
          N > 40ll * current_device_cus();
 }
 
@@ -1354,7 +1358,7 @@ int gemm_launch(const uint16_t* A, int64_t lda, const uint16_t* B, int64_t M, in
   QMOE_REQUIRE(lda % 8 == 0, "qmoe_gemm: lda must be a multiple of 8");
   QMOE_REQUIRE(M < (1ll << 31) && N < (1ll << 31) && K < (1ll << 31), "qmoe_gemm: dims overflow");
   if (M == 0) return QMOE_OK;
-  if (vocab_ok(M, N, K)) {
+  if (vocab_ok(B, M, N, K)) {
     switch (mode) {
       case QMOE_GEMM_STORE_BF16:
         return launch_vocab<QMOE_GEMM_STORE_BF16>(A, lda, B, int(M), int(N), int(K), C, ldc, s);
@@ -1364,7 +1368,7 @@ int gemm_launch(const uint16_t* A, int64_t lda, const uint16_t* B, int64_t M, in
         return launch_vocab<QMOE_GEMM_ADD_F32>(A, lda, B, int(M), int(N), int(K), C, ldc, s);
     }
   }
-  if (skinny_ok(M, N, K) && (M - 1) * lda * 2 + K * 2 < (1ll << 31)) {
+  if (skinny_ok(B, M, N, K) && (M - 1) * lda * 2 + K * 2 < (1ll << 31)) {
     switch (mode) {
       case QMOE_GEMM_STORE_BF16:
         return launch_skinny<QMOE_GEMM_STORE_BF16>(A, lda, B, int(M), int(N), int(K), C, ldc, s);

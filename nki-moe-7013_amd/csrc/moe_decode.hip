@@ -36,7 +36,8 @@ namespace qmoe {
 // whatever the tile: 16 rows x 64 bytes per load are half lines.)
 constexpr int GU_TOK_CHUNK = 4;
 
-template <int HC>
+// DMA = false (x not 16-byte aligned): the copies go through registers.
+template <int HC, bool DMA>
 __global__ __launch_bounds__(256) void moe_gateup_gemv_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ w13,
     const int32_t* __restrict__ offsets, const int32_t* __restrict__ slot_token,
@@ -68,8 +69,11 @@ __global__ __launch_bounds__(256) void moe_gateup_gemv_kernel(
     if (c0 + wave < s1) {  // wave-uniform
 #pragma unroll
       for (int c = 0; c < HC; ++c)
-        pipe::dma16(lds0 + uint32_t(buf * TC * H * 2 + c * 1024), uint32_t(lane * 16),
-                    rx, uint32_t(tok) * uint32_t(H * 2) + uint32_t(c * 1024));
+        if constexpr (DMA)
+          pipe::dma16(lds0 + uint32_t(buf * TC * H * 2 + c * 1024), uint32_t(lane * 16),
+                      rx, uint32_t(tok) * uint32_t(H * 2) + uint32_t(c * 1024));
+        else
+          *reinterpret_cast<u32x4*>(&xs[buf][wave][c * 512 + lane * 8]) = ld16(x + int64_t(tok) * H + c * 512 + lane * 8);
     }
     tok = slot_token[min(c0 + TC + wave, s1 - 1)];
   };
@@ -223,8 +227,12 @@ static int launch_experts(const uint16_t* x, const uint16_t* w13, const uint16_t
   switch (H / 512) {
 #define QMOE_GU(HC)                                                                                  \
   case HC:                                                                                           \
-    hipLaunchKernelGGL(moe_gateup_gemv_kernel<HC>, g1, dim3(256), 0, s, x, w13, offsets, slot_token, \
-                       active, meta, int(T), int(I), act);                                           \
+    if (reinterpret_cast<uintptr_t>(x) % 16 == 0)                                                    \
+      hipLaunchKernelGGL((moe_gateup_gemv_kernel<HC, true>), g1, dim3(256), 0, s, x, w13, offsets,   \
+                         slot_token, active, meta, int(T), int(I), act);                             \
+    else                                                                                             \
+      hipLaunchKernelGGL((moe_gateup_gemv_kernel<HC, false>), g1, dim3(256), 0, s, x, w13, offsets,  \
+                         slot_token, active, meta, int(T), int(I), act);                             \
     break;
     QMOE_GU(1)
     QMOE_GU(2)

@@ -133,3 +133,50 @@ def test_batched_decode_layer(dev, B):
             assert bool(((new - want).abs() <= want.abs() * 2.0 ** -7 + 1e-5).all())
             a[r, :, pos[b0:b1].long()] = e[r, :, pos[b0:b1].long()]
             assert torch.equal(a, e)
+
+
+def _off_by_four_bytes(t):
+    """The same values as ``t`` in storage that is 4-byte but not 16-byte aligned."""
+    buf = torch.empty(t.numel() + 2, dtype=t.dtype, device=t.device)[2:].view(t.shape)
+    buf.copy_(t)
+    assert buf.is_contiguous() and buf.data_ptr() % 16 == 4
+    return buf
+
+
+def test_operands_off_the_dma_alignment(dev):
+    """Rows and weights that are not 16-byte aligned take the register-loading
+    kernels: same values to the fp32 sums' order."""
+    announce("operands off the DMA alignment")
+    g = _gen(dev, 5)
+    x = bf16_randn((12, H), g, dev)
+    for N in (512, 10304):
+        w = bf16_randn((N, H), g, dev, std=0.02)
+        a = ops.gemm(x, w, _lib.GEMM_STORE_F32)
+        b = ops.gemm(_off_by_four_bytes(x), _off_by_four_bytes(w), _lib.GEMM_STORE_F32)
+        torch.cuda.synchronize()
+        # two fp32 sums of 2048 products in different orders
+        bound = (x.double().abs() @ w.double().abs().t()) * (2 * 2048 * 2.0 ** -24)
+        assert bool(((a.double() - b.double()).abs() <= bound).all())
+    xs = bf16_randn((20, H), g, dev)
+    w13 = bf16_randn((4, 128, H), g, dev, std=0.02)
+    w2 = bf16_randn((4, 8, H, 8), g, dev, std=0.02)
+    ids = torch.randint(0, 4, (20, 1), generator=g, device=dev, dtype=torch.int32)
+    route = ops.moe_permute(ids, 4, 128)
+    ya = ops.moe_experts_gemv(xs, w13, w2, route)
+    yb = ops.moe_experts_gemv(_off_by_four_bytes(xs), w13, w2, route)
+    torch.cuda.synchronize()
+    assert torch.equal(ya, yb)
+    wqkv = bf16_randn(((HQ + 2 * HKV) * D, H), g, dev, std=0.02)
+    nw = torch.ones(D, dtype=torch.bfloat16, device=dev)
+    pos = torch.arange(20, device=dev, dtype=torch.int32)
+    cos, sin = rope_tables(D, 20, 1.0e6, dev)
+    got = []
+    for f in (lambda t: t, _off_by_four_bytes):
+        kc = torch.zeros(1, HKV, 20, D, dtype=torch.bfloat16, device=dev)
+        vc = torch.zeros_like(kc)
+        q = ops.qkv_norm_rope(f(xs), f(wqkv), nw, nw, cos, sin, pos, 1, 20, HQ, HKV, kc, vc, 1e-6)
+        got.append((q, kc, vc))
+    torch.cuda.synchronize()
+    for a, b in zip(*got):
+        # one bf16 step, and the fp32 sums' order below it
+        assert bool(((a.float() - b.float()).abs() <= a.float().abs() * 2.0 ** -7 + 1e-5).all())
