@@ -95,6 +95,15 @@ class Attention:
             self._ws[(B, cache.capacity)] = ws
         return ws
 
+    def _skinny_decode(self, x: torch.Tensor, B: int) -> bool:
+        """Whether a decode step past the GEMV's rows projects with ``ops.gemm``.
+        Above 16 rows some of its kernels copy both operands by LDS-DMA (16
+        bytes a lane, 32-bit offsets); ``qkv_norm_rope`` takes operands that are
+        off that alignment, or too large, through registers."""
+        return (0 < B <= FUSED_DECODE_MAX_ROWS and x.shape[1] in ops.SKINNY_K
+                and x.data_ptr() % 16 == 0 and self.wqkv.data_ptr() % 16 == 0
+                and self.wqkv.numel() * self.wqkv.element_size() < 2**31)
+
     def forward(self, x: torch.Tensor, residual: torch.Tensor, positions: torch.Tensor, B: int, S: int,
                 cache: KVCache, rope_cos: torch.Tensor, rope_sin: torch.Tensor, start=0,
                 max_ctx: Optional[int] = None, norm: Optional[tuple] = None,
@@ -107,7 +116,8 @@ class Attention:
         S == 1: decode; row b sees cache entries ``[0, positions[b]]`` (at most
         the first ``max_ctx`` when a context bucket is given), on every path.
         Up to ``FUSED_DECODE_MAX_ROWS`` decode rows the finish runs inside the
-        attention launch (``attn_decode_fused``).
+        attention launch (``attn_decode_fused``), past the GEMV's rows only
+        with 16-byte aligned ``x`` and ``wqkv``.
         ``norm = (rms_w, eps)``: ``x`` is the fp32 residual row itself (B*S == 1)
         and the input RMSNorm is fused into the QKV GEMV.
         ``post_norm = (rms_w, eps)``: returns ``bf16(rmsnorm(residual) * rms_w)``
@@ -116,7 +126,7 @@ class Attention:
         """
         n_ws = ops.qkv_norm_rope_workspace(B * S, x.shape[1], self.n_q, self.n_kv, self.head_dim)
         n_raw = n_ws
-        if S == 1 and n_ws == 0 and 0 < B <= FUSED_DECODE_MAX_ROWS and x.shape[1] in ops.SKINNY_K:
+        if S == 1 and n_ws == 0 and self._skinny_decode(x, B):
             n_raw = B * self.wqkv.shape[0] * 4
         qws = self._ws.get(("qkv", B * S))
         if qws is None or qws.numel() * 4 < n_raw:
