@@ -143,6 +143,67 @@ def _off_by_four_bytes(t):
     return buf
 
 
+def _f64_decode(x, w, cos, sin, pos, cache):
+    """The decode step in 64 bits: o_proj's output and the new key and value rows."""
+    wqkv, wo, qn, kn = (t.double() for t in w)
+    B = x.shape[0]
+    qkv = (x.double() @ wqkv.t()).view(B, HQ + 2 * HKV, D)
+    c, s = (t[pos.long()].double().unsqueeze(1) for t in (cos, sin))
+
+    def finish(t, nw):
+        t = t * torch.rsqrt(t.square().mean(-1, keepdim=True) + 1e-6) * nw
+        lo, hi = t[..., : D // 2], t[..., D // 2 :]
+        return torch.cat([lo * c - hi * s, hi * c + lo * s], dim=-1)
+
+    q, k, v = finish(qkv[:, :HQ], qn), finish(qkv[:, HQ : HQ + HKV], kn), qkv[:, HQ + HKV :]
+    o = torch.empty(B, HQ, D, dtype=torch.float64, device=x.device)
+    for b, n in enumerate(pos.tolist()):
+        kk = torch.cat([cache.k[b, :, :n].double(), k[b].unsqueeze(1)], 1)
+        vv = torch.cat([cache.v[b, :, :n].double(), v[b].unsqueeze(1)], 1)
+        for j in range(HKV):
+            heads = slice(j * (HQ // HKV), (j + 1) * (HQ // HKV))
+            o[b, heads] = (q[b, heads] @ kk[j].t() * D ** -0.5).softmax(-1) @ vv[j]
+    return o.reshape(B, HQ * D) @ wo.t(), k, v
+
+
+# both sides of the row counts where the projection changes kernel (16, 64) and
+# of its row tiles, the same layer with the QKV weights off the DMA alignment
+@pytest.mark.parametrize("B,aligned", [(9, True), (16, True), (17, True), (20, False), (33, True), (48, True),
+                                       (64, True), (64, False), (65, True)])
+def test_batched_decode_layer_against_64_bits(dev, B, aligned):
+    announce(f"batched decode layer in 64 bits B={B} aligned={aligned}")
+    g = _gen(dev, 100 + B)
+    cap = 700
+    w = (bf16_randn(((HQ + 2 * HKV) * D, H), g, dev, std=0.02), bf16_randn((H, HQ * D), g, dev, std=0.02),
+         (1.0 + 0.1 * torch.randn(D, generator=g, device=dev)).to(torch.bfloat16),
+         (1.0 + 0.1 * torch.randn(D, generator=g, device=dev)).to(torch.bfloat16))
+    cos, sin = rope_tables(D, cap, 1.0e6, dev)
+    x = bf16_randn((B, H), g, dev)
+    pos = torch.randint(0, cap, (B,), generator=g, device=dev, dtype=torch.int32)
+    pos[0], pos[1], pos[2], pos[3] = 0, 63, 64, cap - 1
+    cache = KVCache(B, HKV, cap, D, dev)
+    cache.k.normal_(0.0, 1.0, generator=g)
+    cache.v.normal_(0.0, 1.0, generator=g)
+    y, k, v = _f64_decode(x, w, cos, sin, pos, cache)
+    before = cache.k.clone(), cache.v.clone()
+    wqkv = w[0] if aligned else _off_by_four_bytes(w[0])
+    attn = Attention(wqkv, w[2], w[3], w[1], HQ, HKV, D, 1e-6)
+    out = attn.forward(x, torch.zeros(B, H, device=dev), pos, B, 1, cache, cos, sin)
+    torch.cuda.synchronize()
+    # the layer's update alone (no residual in front of it).  q, k, v, the
+    # probabilities and the heads' outputs are each rounded to bf16: 2^-9 / sqrt(3)
+    # of a value at rms, sqrt(5) times that (2.5e-3) of a row together; the bound
+    # is three times as much.  A lost 64-key block of 700 would be 0.3 of the row
+    row = (out.double() - y).norm(dim=1) / y.norm(dim=1)
+    assert float(row.max()) <= 2.0 ** -7, f"{float(row.max()):.2e}"
+    rows = torch.arange(B, device=dev)
+    for a, b, want in ((cache.k, before[0], k), (cache.v, before[1], v)):
+        err = (a[rows, :, pos.long()].double() - want).abs() - want.abs() * 2.0 ** -8
+        assert float(err.max()) <= 2e-4  # one bf16 rounding, and the fp32 sums below it
+        a[rows, :, pos.long()] = b[rows, :, pos.long()]
+        assert torch.equal(a, b)  # no other row of the cache is written
+
+
 def test_operands_off_the_dma_alignment(dev):
     """Rows and weights that are not 16-byte aligned take the register-loading
     kernels: same values to the fp32 sums' order."""
