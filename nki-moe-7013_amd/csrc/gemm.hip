@@ -1207,20 +1207,42 @@ static int launch_gemv_pk(const uint16_t* A, int64_t lda, const uint16_t* B, int
   return fail(QMOE_ERR_INVALID, "qmoe_gemm: packed GEMV needs K in {512, 1024, 2048, 4096}");
 }
 
-// B is copied by LDS-DMA, 16 bytes a lane: a B that is not 16-byte aligned
-// stays on the kernels that load it into registers.
+// The skinny and vocabulary kernels copy B by LDS-DMA, 16 bytes a lane; a B
+// that is not 16-byte aligned stays on the kernels of the general order: the
+// 9 to 16 rows of those load it into registers, the others (packed GEMV, MFMA
+// tiles) copy it by LDS-DMA too.
 static bool dma_aligned(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
-// Rows and shapes that gemm_skinny_kernel takes: up to two rounds of its
-// 20-column workgroups.  Measured against the kernels that took these shapes
-// before (16-row GEMV, 64 x 64 tiles), 9 / 16 / 32 / 64 rows: N = 5120, K =
-// 2048 8.9 / 11.5 / 12.1 / 13.0 -> 6.2 / 6.9 / 8.8 / 12.5 us; N = 2048, K =
-// 4096 20.5 / 20.8 / 21.8 / 23.1 -> 6.5 / 7.8 / 10.9 / 18.2 us.  At the
-// vocabulary's N = 151936 every one of 7597 workgroups re-reads A (148 / 222 /
-// 314 us at 12 / 32 / 64 rows): gemm_vocab_kernel's.
-static bool skinny_ok(const void* B, int64_t M, int64_t N, int64_t K) {
-  return dma_aligned(B) && M >= 9 && M <= 64 && (K == 512 || K == 1024 || K == 2048 || K == 4096) && N * K * 2 < (1ll << 31) &&
-         N <= 40ll * current_device_cus();
+// Columns per workgroup of gemm_skinny_kernel, 0 where another kernel takes
+// the shape.  Every workgroup reads all of A from L2 and runs every row tile,
+// so the fewest columns that give each CU at most one workgroup are taken
+// (N = 1536, K = 2048 at 16 / 48 rows on 8 columns 4.6 / 8.1 us, on 4 and
+// twice the workgroups 6.6 / 13.0).  us against the kernels that had these
+// shapes before (16-row GEMV up to 16 rows of K <= 2048, 64 x 64 tiles), at 9 /
+// 16 / 32 / 64 rows:
+//   N = 5120, K = 2048   8.9 / 11.5 / 12.1 / 12.8 -> 6.2 / 6.9 / 9.1 / 12.4
+//   N = 2048, K = 4096   20.1 / 20.1 / 20.4 / 21.5 -> 6.1 / 7.3 / 10.5 / 17.6
+// A short K leaves a wave so little to do that the columns of 20 (two MFMA
+// column tiles) and the last row tile lose: N = 5120, K = 1024 at 40 rows 7.2 ->
+// 8.3, K = 512 at 17 rows 4.8 -> 5.3; N = 4096, K = 512 at 64 rows 5.0 -> 5.4.
+// A second round of workgroups wins up to 16 rows once it is about half full
+// (N = 7168, K = 2048, 9 / 16 rows 10.4 / 14.1 -> 9.9 / 11.4; N = 6144 at 9
+// rows 9.1 -> 9.7) and loses above (N = 8192, 17 / 64 rows 12.2 / 13.4 -> 14.4
+// / 22.6); where the others are slow, at K = 4096, it wins from its start and
+// up to 24 rows (N = 8192 at 24 / 32 rows 23.1 / 23.4 -> 21.5 / 24.1; N =
+// 10240, two and a half rounds, at 12 / 17 rows 25.2 / 25.4 -> 22.9 / 26.8).
+static int skinny_cols(const void* B, int64_t M, int64_t N, int64_t K) {
+  if (!dma_aligned(B) || M < 9 || M > 64 || (K != 512 && K != 1024 && K != 2048 && K != 4096) ||
+      N * K * 2 >= (1ll << 31))
+    return 0;
+  const int64_t cus = current_device_cus();
+  for (int nb : {4, 8, 16, 20}) {
+    if (N > nb * cus || (nb == 20 && K == 4096)) continue;  // 20 columns of 4096 do not fit in LDS
+    const int64_t rows = nb == 20 ? (K == 512 ? 16 : K == 1024 ? 32 : 64) : (K == 512 ? 48 : 64);
+    return M <= rows ? nb : 0;
+  }
+  if (K == 4096) return M <= (N <= 32 * cus ? 24 : N <= 40 * cus ? 16 : 0) ? 16 : 0;
+  return K >= 1024 && M <= 16 && N >= 28 * cus && N <= 40 * cus ? 20 : 0;
 }
 
 // Rows and shapes of gemm_vocab_kernel: the column counts above the skinny
@@ -1285,11 +1307,8 @@ static int launch_skinny_t(const uint16_t* A, int64_t lda, const uint16_t* B, in
 }
 
 template <int MODE>
-static int launch_skinny(const uint16_t* A, int64_t lda, const uint16_t* B, int M, int N, int K, void* C,
+static int launch_skinny(int nb, const uint16_t* A, int64_t lda, const uint16_t* B, int M, int N, int K, void* C,
                          int64_t ldc, hipStream_t s) {
-  // columns per workgroup by the rule of the packed GEMV
-  const int cus = current_device_cus();
-  const int nb = N >= 20 * cus && K <= 2048 ? 20 : N >= 16 * cus ? 16 : N >= 8 * cus ? 8 : 4;
 #define QMOE_SK(W, NB_)                                                                            \
   if (K == 512 * W && nb == NB_)                                                                   \
     return M <= 16   ? launch_skinny_t<W, NB_, 1, MODE>(A, lda, B, M, N, K, C, ldc, s)              \
@@ -1368,14 +1387,14 @@ int gemm_launch(const uint16_t* A, int64_t lda, const uint16_t* B, int64_t M, in
         return launch_vocab<QMOE_GEMM_ADD_F32>(A, lda, B, int(M), int(N), int(K), C, ldc, s);
     }
   }
-  if (skinny_ok(B, M, N, K) && (M - 1) * lda * 2 + K * 2 < (1ll << 31)) {
+  if (const int nb = skinny_cols(B, M, N, K); nb && (M - 1) * lda * 2 + K * 2 < (1ll << 31)) {
     switch (mode) {
       case QMOE_GEMM_STORE_BF16:
-        return launch_skinny<QMOE_GEMM_STORE_BF16>(A, lda, B, int(M), int(N), int(K), C, ldc, s);
+        return launch_skinny<QMOE_GEMM_STORE_BF16>(nb, A, lda, B, int(M), int(N), int(K), C, ldc, s);
       case QMOE_GEMM_STORE_F32:
-        return launch_skinny<QMOE_GEMM_STORE_F32>(A, lda, B, int(M), int(N), int(K), C, ldc, s);
+        return launch_skinny<QMOE_GEMM_STORE_F32>(nb, A, lda, B, int(M), int(N), int(K), C, ldc, s);
       default:
-        return launch_skinny<QMOE_GEMM_ADD_F32>(A, lda, B, int(M), int(N), int(K), C, ldc, s);
+        return launch_skinny<QMOE_GEMM_ADD_F32>(nb, A, lda, B, int(M), int(N), int(K), C, ldc, s);
     }
   }
   if (M <= 16 && M * K <= 32768) {

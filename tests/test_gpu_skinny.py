@@ -18,10 +18,13 @@ def _gen(dev, seed):
     return torch.Generator(device=dev).manual_seed(seed)
 
 
-# every row-tile count and its edges; column remainders of the 4-, 8-, 16- and
-# 20-column workgroups and of the 64-column slices; every K
-@pytest.mark.parametrize("M", [9, 16, 17, 32, 33, 48, 49, 64])
-@pytest.mark.parametrize("N,K", [(5120, 2048), (2048, 4096), (1111, 512), (4133, 1024), (5129, 1024), (64, 2048)])
+# every row-tile count and its edges; every K; column remainders of the 4-, 8-,
+# 16- and 20-column workgroups (up to 1024, 2048, 4096 and 5120 columns on 256
+# CUs) and of their second round (7181; 4133 at K = 4096)
+@pytest.mark.parametrize("M", [9, 16, 17, 24, 32, 33, 48, 49, 64])
+@pytest.mark.parametrize("N,K", [(5120, 2048), (2048, 4096), (1111, 512), (4133, 1024), (5129, 1024), (64, 2048),
+                                 (1023, 512), (1021, 4096), (1301, 2048), (2051, 1024), (4133, 2048), (4609, 512),
+                                 (4133, 4096), (7181, 2048), (7181, 1024)])
 def test_skinny_gemm(dev, M, N, K):
     announce(f"skinny gemm M={M} N={N} K={K}")
     g = _gen(dev, M * 7 + N)
@@ -43,6 +46,23 @@ def test_skinny_gemm(dev, M, N, K):
         assert torch.equal(c, again)
         assert torch.equal(cb, c.to(torch.bfloat16))
         assert torch.equal(acc, base + c)
+
+
+# Shapes at which the 64 x 64 tiles are ahead of the skinny kernel (a second
+# round of its workgroups, the wide workgroups and the fourth row tile at a
+# short K).  The tiles sum K in one chain, so their rows carry the bits of the
+# same rows in a product of more rows than the skinny kernel takes.
+@pytest.mark.parametrize("M,N,K", [(17, 5632, 2048), (48, 6144, 2048), (64, 10240, 2048), (33, 5120, 1024),
+                                   (64, 9216, 1024), (25, 8192, 4096), (17, 10240, 4096)])
+def test_tiles_keep_their_shapes(dev, M, N, K):
+    announce(f"tiles M={M} N={N} K={K}")
+    g = _gen(dev, M + N)
+    A = bf16_randn((65, K), g, dev)
+    B = bf16_randn((N, K), g, dev, std=0.05)
+    c = ops.gemm(A[:M].contiguous(), B, _lib.GEMM_STORE_F32)
+    ref = ops.gemm(A, B, _lib.GEMM_STORE_F32)[:M]
+    torch.cuda.synchronize()
+    assert torch.equal(c, ref)
 
 
 # the vocabulary kernel: row-tile edges, a last tile of one column, fewer and
