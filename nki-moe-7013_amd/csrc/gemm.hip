@@ -350,12 +350,22 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_pk_kernel(const uint16_t* __r
 // straight from global memory, the next tile's in flight behind this one's
 // MFMAs.  Bound by the weight stream plus the A rows that every workgroup
 // re-reads from L2 (M * K * 2 bytes, 1-4 us of a CU's L2 port).
+// Up to 16 rows K is summed in at least the four chains of gemv_mfma_kernel,
+// quarter by quarter and added in order: the same bits, where one chain per
+// wave was further from the exact sum at K = 512 (1.25e-7 against 0.72e-7 of
+// its norm) and 1024 (1.27e-7 against 0.95e-7), at the same time (N = 4096 at
+// 16 rows: 3.4 and 3.9 us).
+template <int WAVES, int MT>
+struct Skinny {
+  static constexpr int CHAINS = MT == 1 && WAVES < 4 ? 4 / WAVES : 1;  // of each wave
+};
 template <int WAVES, int NB, int MT, int MODE>
 __global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(const uint16_t* __restrict__ A, int64_t lda,
                                                                  const uint16_t* __restrict__ B, int M, int N,
                                                                  int K, void* __restrict__ C, int64_t ldc) {
   constexpr int NT = (NB + 15) / 16;  // 16-column MFMA tiles
   constexpr int RLD = NB + 1;
+  constexpr int CH = Skinny<WAVES, MT>::CHAINS, PARTS = WAVES * CH;
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];  // weights; then the partials
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -383,11 +393,13 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(const uint16_t*
     }
   }
   pipe::wait_vm<0>();  // this wave's weight rows are in LDS (and its first A tile in registers)
-  f32x4 acc[MT][NT];
+  f32x4 acc[MT][NT][CH];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{};
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int c = 0; c < CH; ++c) acc[i][j][c] = f32x4{};
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
     if (i + 1 < MT) load_a(af[(i + 1) & 1], i + 1);
@@ -396,27 +408,31 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_skinny_kernel(const uint16_t*
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
         const u32x4 b = *reinterpret_cast<const u32x4*>(wl + min(j * 16 + col, NB - 1) * GV_ROWB + kg * 16 + s * 64);
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, af[i & 1][s]),
-                                                            __builtin_bit_cast(bf16x8, b), acc[i][j], 0, 0, 0);
+        f32x4& a = acc[i][j][s * CH / 16];
+        a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, af[i & 1][s]),
+                                                    __builtin_bit_cast(bf16x8, b), a, 0, 0, 0);
       }
   }
   // lane l holds column l % 16 of tile j, rows 16 i + (l / 16) * 4 + 0..3
   __syncthreads();  // the weights are used up: their LDS takes the partials
-  float* red = reinterpret_cast<float*>(smem);  // [WAVES][MT * 16][RLD]
+  float* red = reinterpret_cast<float*>(smem);  // [PARTS][MT * 16][RLD]
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
     for (int j = 0; j < NT; ++j)
       if (j * 16 + col < NB)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) red[(wave * MT * 16 + i * 16 + kg * 4 + e) * RLD + j * 16 + col] = acc[i][j][e];
+        for (int c = 0; c < CH; ++c)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            red[((wave * CH + c) * MT * 16 + i * 16 + kg * 4 + e) * RLD + j * 16 + col] = acc[i][j][c][e];
   __syncthreads();
   for (int i = t; i < min(M, MT * 16) * NB; i += 64 * WAVES) {
     const int m = i / NB, n = i % NB;
     if (n0 + n < N) {
       float v = red[m * RLD + n];
 #pragma unroll
-      for (int w = 1; w < WAVES; ++w) v += red[(w * MT * 16 + m) * RLD + n];
+      for (int p = 1; p < PARTS; ++p) v += red[(p * MT * 16 + m) * RLD + n];
       store_out<MODE>(C, int64_t(m) * ldc + n0 + n, v);
     }
   }
@@ -1292,7 +1308,7 @@ static int launch_vocab(const uint16_t* A, int64_t lda, const uint16_t* B, int M
 template <int WAVES, int NB, int MT, int MODE>
 static int launch_skinny_t(const uint16_t* A, int64_t lda, const uint16_t* B, int M, int N, int K, void* C,
                            int64_t ldc, hipStream_t s) {
-  constexpr int W_BYTES = WAVES * NB * GV_ROWB, R_BYTES = WAVES * MT * 16 * (NB + 1) * 4;
+  constexpr int W_BYTES = WAVES * NB * GV_ROWB, R_BYTES = WAVES * Skinny<WAVES, MT>::CHAINS * MT * 16 * (NB + 1) * 4;
   constexpr int SMEM = W_BYTES > R_BYTES ? W_BYTES : R_BYTES;
   static_assert(SMEM <= 160 * 1024, "LDS");
   static const bool attr = [] {

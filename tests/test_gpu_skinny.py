@@ -65,6 +65,24 @@ def test_tiles_keep_their_shapes(dev, M, N, K):
     assert torch.equal(c, ref)
 
 
+# The sum over K keeps the accuracy of four chains up to 16 rows.  Rounding a
+# chain of n of the K / 32 steps after each one walks n (n + 1) / 2 / (K / 32)
+# steps of (2^-24)^2 / 3 of the final variance, and adding four chains 2.25 more:
+# 7.5e-8 of the norm at K = 512 and 8.9e-8 at 1024 (one and two chains: 1.0e-7
+# and 1.06e-7 at least).  The bound leaves a quarter on top
+@pytest.mark.parametrize("K,walk", [(512, 7.5e-8), (1024, 8.9e-8)])
+@pytest.mark.parametrize("M", [9, 16])
+def test_skinny_sum_accuracy(dev, M, K, walk):
+    announce(f"skinny sum accuracy M={M} K={K}")
+    g = _gen(dev, K + M)
+    A = bf16_randn((M, K), g, dev)
+    B = bf16_randn((4096, K), g, dev, std=0.05)
+    c = ops.gemm(A, B, _lib.GEMM_STORE_F32)
+    ref = A.double() @ B.double().t()
+    torch.cuda.synchronize()
+    assert float((c.double() - ref).norm() / ref.norm()) <= 1.25 * walk
+
+
 # the vocabulary kernel: row-tile edges, a last tile of one column, fewer and
 # more tiles than a round of workgroups, both K
 @pytest.mark.parametrize("M", [2, 8, 9, 16, 17, 33, 48, 64])
