@@ -451,11 +451,18 @@ constexpr int VO_S = 2, VO_TILE = 16 * 512;
 // Row m of a partial tile sits at vo_row(m): the four lane groups' rows (4
 // apart) are neighbours, so their stores and the sums' reads hit all banks.
 __device__ __forceinline__ int vo_row(int m) { return (m & ~15) | ((m & 3) << 2) | ((m >> 2) & 3); }
+// 8 waves fill a CU: two workgroups of 4 waves (K = 1024) share it, so the
+// second set of partial tiles (one barrier less per tile) is taken only where
+// both still fit.  With it, 33 rows and more of K = 1024 left one workgroup per
+// CU and half of the launch waiting (N = 40000, 33 / 64 rows 21.3 / 26.4 us,
+// 18.9 / 23.8 on one set).
 template <int WAVES, int MT>
 struct Vocab {
+  static constexpr int PER_CU = 8 / WAVES, LDS = 160 * 1024 / PER_CU;  // workgroups of a CU, LDS of each
   static constexpr int RED = WAVES * MT * 256 * 4;  // bytes of one set of partial tiles
-  static constexpr int NRED = WAVES * VO_S * VO_TILE + 2 * RED <= 160 * 1024 ? 2 : 1;
+  static constexpr int NRED = WAVES * VO_S * VO_TILE + 2 * RED <= LDS ? 2 : 1;
   static constexpr int SMEM = WAVES * VO_S * VO_TILE + NRED * RED;
+  static_assert(SMEM <= LDS, "LDS");
 };
 template <int WAVES, int MT, int MODE>
 __global__ __launch_bounds__(64 * WAVES) void gemm_vocab_kernel(const uint16_t* __restrict__ A, int64_t lda,
@@ -1261,29 +1268,42 @@ static int skinny_cols(const void* B, int64_t M, int64_t N, int64_t K) {
   return K >= 1024 && M <= 16 && N >= 28 * cus && N <= 40 * cus ? 20 : 0;
 }
 
-// Rows and shapes of gemm_vocab_kernel: the column counts above the skinny
-// kernel's.  N = 151936, K = 2048 at 2 / 8 / 16 / 32 / 64 rows, against the
-// packed GEMV, the 16-row GEMV and the 256 x 256 tiles: 118 / 131 / 149 / 159 /
-// 169 -> 102 / 109 / 116 / 122 / 132 us (6.1 to 4.7 TB/s, of which the fp32
-// output takes 1 to 39 MB); N = 20000, K = 1024, 32 rows 19.4 -> 11.6 us.  At K = 512 a
-// tile is too short for its barrier (N = 10243, 33 rows: 5.1 -> 6.8 us).
+// Rows and shapes of gemm_vocab_kernel: more than the skinny kernel's columns.
+// N = 151936, K = 2048 at 2 / 8 / 16 / 32 / 64 rows, against the packed GEMV,
+// the 16-row GEMV and the 256 x 256 tiles: 118 / 131 / 149 / 159 / 174 -> 102 /
+// 109 / 116 / 122 / 132 us (6.1 to 4.7 TB/s, of which the fp32 output takes 1
+// to 39 MB); N = 20000, K = 1024, 32 rows 19.4 -> 11.7 us.  The others stay
+// ahead, and have the shape,
+//   - above 24 rows while the 64 x 64 tiles are used (fewer than 96 column
+//     tiles of 128; at 24 / 32 / 64 rows N = 12160 runs 14.3 / 14.7 / 15.2 us
+//     there and 14.2 / 14.9 / 19.8 here at K = 2048, 7.9 / 8.2 / 8.7 and 7.7 /
+//     8.6 / 12.8 at K = 1024);
+//   - at K = 1024, above 48 rows while the 256 x 256 tiles make one full round
+//     (N = 65536 at 64 rows 32.3 against 33.9 us), and up to 4 rows past 400
+//     columns per CU (packed GEMV; N = 151936 at 2 rows 49.1 against 50.1);
+//   - at K = 512, where a tile is too short for its barrier (N = 10243, 33
+//     rows: 5.1 against 6.8 us).
+// At K = 4096 the 16-wave form does not fit a CU's LDS: its ring alone is 256 KB.
 static bool vocab_ok(const void* B, int64_t M, int64_t N, int64_t K) {
-  return dma_aligned(B) && M >= 2 && M <= 64 && (K == 1024 || K == 2048) && N * K * 2 < (1ll << 31) &&
-         N > 40ll * current_device_cus();
+  const int64_t cus = current_device_cus(), wide = (N + 255) / 256;
+  if (!dma_aligned(B) || M < 2 || M > 64 || (K != 1024 && K != 2048) || N * K * 2 >= (1ll << 31) || N <= 40 * cus)
+    return false;
+  if ((N + 127) / 128 < 96) return M <= 24;
+  if (K == 1024) return !(M > 48 && wide >= 224 && wide <= cus) && !(M <= 4 && N > 400 * cus);
+  return true;
 }
 
 template <int WAVES, int MT, int MODE>
 static int launch_vocab_t(const uint16_t* A, int64_t lda, const uint16_t* B, int M, int N, int K, void* C,
                           int64_t ldc, hipStream_t s) {
   constexpr int SMEM = Vocab<WAVES, MT>::SMEM;
-  static_assert(SMEM <= 160 * 1024, "LDS");
   static const bool attr = [] {
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_vocab_kernel<WAVES, MT, MODE>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, SMEM);
     return true;
   }();
   (void)attr;
-  const int64_t groups = int64_t(std::max(current_device_cus(), 1)) * (8 / WAVES);
+  const int64_t groups = int64_t(std::max(current_device_cus(), 1)) * Vocab<WAVES, MT>::PER_CU;
   hipLaunchKernelGGL((gemm_vocab_kernel<WAVES, MT, MODE>), dim3(unsigned(std::min<int64_t>((N + 15) / 16, groups))),
                      dim3(64 * WAVES), SMEM, s, A, lda, B, M, N, K, C, ldc);
   return hip_status("qmoe_gemm(vocab)");

@@ -50,10 +50,11 @@ def test_skinny_gemm(dev, M, N, K):
 
 # Shapes at which the 64 x 64 tiles are ahead of the skinny kernel (a second
 # round of its workgroups, the wide workgroups and the fourth row tile at a
-# short K).  The tiles sum K in one chain, so their rows carry the bits of the
+# short K) or of the vocabulary kernel (its first columns, from 25 rows).  The tiles sum K in one chain, so their rows carry the bits of the
 # same rows in a product of more rows than the skinny kernel takes.
 @pytest.mark.parametrize("M,N,K", [(17, 5632, 2048), (48, 6144, 2048), (64, 10240, 2048), (33, 5120, 1024),
-                                   (64, 9216, 1024), (25, 8192, 4096), (17, 10240, 4096)])
+                                   (64, 9216, 1024), (25, 8192, 4096), (17, 10240, 4096), (25, 10244, 1024),
+                                   (64, 12160, 1024), (32, 12160, 2048)])
 def test_tiles_keep_their_shapes(dev, M, N, K):
     announce(f"tiles M={M} N={N} K={K}")
     g = _gen(dev, M + N)
@@ -83,10 +84,12 @@ def test_skinny_sum_accuracy(dev, M, K, walk):
     assert float((c.double() - ref).norm() / ref.norm()) <= 1.25 * walk
 
 
-# the vocabulary kernel: row-tile edges, a last tile of one column, fewer and
-# more tiles than a round of workgroups, both K
-@pytest.mark.parametrize("M", [2, 8, 9, 16, 17, 33, 48, 64])
-@pytest.mark.parametrize("N,K", [(10241, 2048), (12289, 1024), (40001, 2048)])
+# the vocabulary kernel: row-tile edges, a last tile of one column, one to five
+# tiles per workgroup (from the third on the ring's slots are filled again) and
+# both K
+@pytest.mark.parametrize("M", [2, 8, 9, 16, 17, 24, 33, 48, 64])
+@pytest.mark.parametrize("N,K", [(10241, 2048), (12289, 1024), (40001, 2048), (12161, 1024), (40001, 1024),
+                                 (20002, 1024), (20003, 2048)])
 def test_vocab_gemm(dev, M, N, K):
     test_skinny_gemm(dev, M, N, K)
 
