@@ -52,26 +52,27 @@ __device__ __forceinline__ uint64_t block_max_u64(uint64_t k, uint64_t* red) {
   return m;
 }
 
-// Workgroup (slice p of gridDim.x, row): AM_U values per thread in flight.
-// Many rows take fewer, longer slices (argmax_parts): with 256 slices a row,
-// 32 rows of 151,936 were 8192 workgroups of two loads a thread, one after
-// the other: 13 us for 19 MB.
-constexpr int AM_U = 8;
+// Workgroup (slice p of `chunk` values, row): U values per thread in flight, as
+// many as the slice has for a thread, up to 8 (with a fixed 8, and the slice's
+// length divided out in each thread, 2 rows of 20,000 took 4.9 us with the final
+// pass instead of 4.5).  Many rows take fewer, longer slices (qmoe_argmax): with
+// 256 slices a row, 32 rows of 151,936 were 8192 workgroups of two loads a
+// thread, one after the other: 13 us for 19 MB.
+template <int U>
 __global__ __launch_bounds__(ARGMAX_THREADS) void argmax_partial_kernel(const float* __restrict__ x,
-                                                                        int64_t n, int64_t ldx,
+                                                                        int64_t n, int64_t ldx, int64_t chunk,
                                                                         uint64_t* __restrict__ part) {
   __shared__ uint64_t red[ARGMAX_THREADS / 64];
   const int row = blockIdx.y, p = blockIdx.x;
-  const int64_t chunk = (n + gridDim.x - 1) / gridDim.x;
   const int64_t b0 = int64_t(p) * chunk, b1 = min(n, b0 + chunk);
   const float* xr = x + int64_t(row) * ldx;
   uint64_t k = 0;  // below every real key (index complement of -1 never wins)
-  for (int64_t i = b0 + threadIdx.x; i < b1; i += ARGMAX_THREADS * AM_U) {
-    float v[AM_U];
+  for (int64_t i = b0 + threadIdx.x; i < b1; i += ARGMAX_THREADS * U) {
+    float v[U];
 #pragma unroll
-    for (int u = 0; u < AM_U; ++u) v[u] = xr[min(i + u * ARGMAX_THREADS, b1 - 1)];
+    for (int u = 0; u < U; ++u) v[u] = xr[min(i + u * ARGMAX_THREADS, b1 - 1)];
 #pragma unroll
-    for (int u = 0; u < AM_U; ++u)  // a value past the slice is its last one again: the same key
+    for (int u = 0; u < U; ++u)  // a value past the slice is its last one again: the same key
       k = u64max(k, argmax_key(v[u], min(i + u * ARGMAX_THREADS, b1 - 1)));
   }
   k = block_max_u64(k, red);
@@ -126,8 +127,12 @@ extern "C" int qmoe_argmax(const float* x, int64_t rows, int64_t n, int64_t ldx,
   uint64_t* part = static_cast<uint64_t*>(workspace);
   // slices of a row: all 256 for a few rows, then about 1024 workgroups, at least 8 a row
   const int parts = int(std::min<int64_t>(ARGMAX_PARTS, std::max<int64_t>(8, 1024 / rows)));
-  hipLaunchKernelGGL(argmax_partial_kernel, dim3(parts, unsigned(rows)), dim3(ARGMAX_THREADS), 0,
-                     s, x, n, ldx, part);
+  const int64_t chunk = (n + parts - 1) / parts, per_thread = (chunk + ARGMAX_THREADS - 1) / ARGMAX_THREADS;
+  const auto partial = per_thread <= 1   ? argmax_partial_kernel<1>
+                       : per_thread <= 2 ? argmax_partial_kernel<2>
+                       : per_thread <= 4 ? argmax_partial_kernel<4>
+                                         : argmax_partial_kernel<8>;
+  hipLaunchKernelGGL(partial, dim3(parts, unsigned(rows)), dim3(ARGMAX_THREADS), 0, s, x, n, ldx, chunk, part);
   if (int rc = hip_status("qmoe_argmax(partial)")) return rc;
   hipLaunchKernelGGL(argmax_final_kernel, dim3(unsigned(rows)), dim3(ARGMAX_THREADS), 0, s, part, parts, out);
   return hip_status("qmoe_argmax(final)");

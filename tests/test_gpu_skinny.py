@@ -95,8 +95,11 @@ def test_vocab_gemm(dev, M, N, K):
 
 
 # every slice count of the partial pass (256, 34, 8), slices longer and shorter
-# than a thread's eight values, rows of one value
-@pytest.mark.parametrize("rows,n", [(1, 1), (3, 255), (4, 151936), (30, 20011), (64, 151936), (130, 4097), (300, 7)])
+# than a thread's eight values, rows of one value; both sides of the slice
+# lengths of one, two, four and eight values a thread (256, 512, 1024)
+@pytest.mark.parametrize("rows,n", [(1, 1), (3, 255), (4, 151936), (30, 20011), (64, 151936), (130, 4097), (300, 7),
+                                    (4, 65536), (4, 65537), (4, 131072), (4, 131073), (4, 262144), (4, 262145),
+                                    (3, 600000)])
 def test_argmax_slices(dev, rows, n):
     announce(f"argmax rows={rows} n={n}")
     g = _gen(dev, rows + n)
