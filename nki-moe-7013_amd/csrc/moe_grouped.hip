@@ -29,6 +29,7 @@
 // items from per-XCD queues; see the queue helpers below.  Both GEMMs run in
 // one launch (moe_experts_fused_kernel) when the act rows are whole cache
 // lines, else as two launches.
+#include <algorithm>
 #include <atomic>
 
 #include "mfma_wide.hpp"
@@ -50,10 +51,15 @@ using ColdNt = pipe::Wide<4, 2, 64, 4, 64, true>;
 using Warm = pipe::Wide<4, 2, 64, 3, 128>;
 using WarmNt = pipe::Wide<4, 2, 64, 3, 128, true>;
 constexpr int COLD_MAX_ROWS = Cold::BN, WARM_MAX_ROWS = Warm::BN;
-constexpr int PIPE_SMEM = Hot::SMEM > Cold::SMEM ? Hot::SMEM : Cold::SMEM;
+constexpr int PIPE_SMEM = std::max({Hot::SMEM, Cold::SMEM, Warm::SMEM});
 constexpr int PANEL = Hot::BM;
-static_assert(Hot::BM == Cold::BM && Hot::THREADS == Cold::THREADS, "one grid for both pipelines");
-static_assert(Cold::BK % QMOE_W2_BLOCK == 0 && Hot::BK % QMOE_W2_BLOCK == 0, "a stage covers whole w2 blocks");
+static_assert(Hot::BM == Cold::BM && Hot::BM == Warm::BM && Hot::THREADS == Cold::THREADS &&
+                  Hot::THREADS == Warm::THREADS,
+              "one grid for the three pipelines");
+static_assert(Cold::BK % QMOE_W2_BLOCK == 0 && Warm::BK % QMOE_W2_BLOCK == 0 && Hot::BK % QMOE_W2_BLOCK == 0,
+              "a stage covers whole w2 blocks");
+static_assert(Warm::BK == Cold::BK && Cold::BK % Hot::BK == 0, "down_item tests I against one BK");
+static_assert(ColdNt::SMEM == Cold::SMEM && WarmNt::SMEM == Warm::SMEM, "the non-temporal forms share the layout");
 static_assert(PANEL % (2 * QMOE_W13_GROUP) == 0 && QMOE_W13_GROUP == 32,
               "a wave's 64 packed w13 rows are one gate block and its up block");
 
