@@ -66,6 +66,27 @@ def test_tiles_keep_their_shapes(dev, M, N, K):
     assert torch.equal(c, ref)
 
 
+# the slices of the split-K plans of 512 columns (two, four and eight of them) on
+# 64-column tiles whose last one is partial, at each row-tile count, against
+# 64 bits (the comparison is test_skinny_gemm's), and with the norm in the reduction
+@pytest.mark.parametrize("M", [17, 32, 33, 48, 49, 64])
+@pytest.mark.parametrize("N,K", [(2000, 4096), (1924, 4096), (4004, 2048), (5004, 1024)])
+def test_slice_remainders(dev, M, N, K):
+    ws = ops.gemm_workspace(M, N, K, dev)
+    assert ws is not None and ws.numel() == K // 512 * M * N and -(-N // 64) * (K // 512) <= 256
+    test_skinny_gemm(dev, M, N, K)
+    g = _gen(dev, M + N + K)
+    A = bf16_randn((M, K), g, dev)
+    B = bf16_randn((N, K), g, dev, std=0.05)
+    w = bf16_randn((N,), g, dev)
+    h = torch.randn(M, N, generator=g, device=dev)
+    want = ops.gemm(A, B, _lib.GEMM_ADD_F32, out=h.clone(), workspace=ws)
+    x = ops.gemm_add_rmsnorm(A, B, h, w, 1e-6, workspace=ws)
+    torch.cuda.synchronize()
+    assert torch.equal(h, want)
+    assert torch.equal(x, ops.rmsnorm_residual(h, w, 1e-6))
+
+
 # The sum over K keeps the accuracy of four chains up to 16 rows.  Rounding a
 # chain of n of the K / 32 steps after each one walks n (n + 1) / 2 / (K / 32)
 # steps of (2^-24)^2 / 3 of the final variance, and adding four chains 2.25 more:
@@ -246,6 +267,35 @@ def test_batched_decode_layer_against_64_bits(dev, B, aligned):
         assert float(err.max()) <= 2e-4  # one bf16 rounding, and the fp32 sums below it
         a[rows, :, pos.long()] = b[rows, :, pos.long()]
         assert torch.equal(a, b)  # no other row of the cache is written
+
+
+def _off_by(t, nbytes):
+    """The same values as ``t``, ``nbytes`` past a 16-byte boundary."""
+    buf = torch.empty(t.numel() + 8, dtype=t.dtype, device=t.device)[nbytes // 2 :][: t.numel()].view(t.shape)
+    buf.copy_(t)
+    assert buf.is_contiguous() and buf.data_ptr() % 16 == nbytes
+    return buf
+
+
+# every GEMM of few rows (packed and 16-row GEMV, tiles, split K), each operand
+# off the 16-byte boundary by each whole dword
+@pytest.mark.parametrize("M", [1, 2, 8, 9, 16, 17, 64])
+@pytest.mark.parametrize("N,K", [(512, 2048), (10304, 2048), (2048, 4096), (2050, 1024)])
+def test_gemm_off_the_dma_alignment(dev, M, N, K):
+    announce(f"gemm off the DMA alignment M={M} N={N} K={K}")
+    g = _gen(dev, M + N)
+    A = bf16_randn((M, K), g, dev)
+    B = bf16_randn((N, K), g, dev, std=0.05)
+    ref = A.double() @ B.double().t()
+    # fp32 sums of K products in any order: K * 2^-24 of the sum of magnitudes
+    bound = (A.double().abs() @ B.double().abs().t()).mul_(K * 2.0 ** -24)
+    ws = ops.gemm_workspace(M, N, K, dev)
+    for oa, ob in ((4, 0), (0, 4), (8, 8), (12, 4)):
+        a, b = (_off_by(t, o) if o else t for t, o in ((A, oa), (B, ob)))
+        for w in (None, ws) if ws is not None else (None,):
+            c = ops.gemm(a, b, _lib.GEMM_STORE_F32, workspace=w)
+            torch.cuda.synchronize()
+            assert bool(((c.double() - ref).abs() <= bound).all()), (oa, ob, w is not None)
 
 
 def test_operands_off_the_dma_alignment(dev):
