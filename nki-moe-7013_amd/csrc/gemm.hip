@@ -7,8 +7,9 @@
 //    non-temporal loads (K/512 loads per row per lane, all in flight), and
 //    reduces the per-lane partial dots with cross-lane shuffles.
 //  * 9 <= M <= 64 (batched decode, from 2 rows at vocabulary-size N): the
-//    weights stream through LDS past the rows (gemm_skinny_kernel,
-//    gemm_slice_kernel, gemm_vocab_kernel).
+//    weights stream through LDS past the rows, where that is ahead
+//    (gemm_skinny_kernel: skinny_cols, gemm_slice_kernel: slice_ok,
+//    gemm_vocab_kernel: vocab_ok).
 //  * larger M: the direct-to-LDS MFMA pipelines (mfma_pipe.hpp; from 224
 //    tiles of 256 x 256 on, the deep-staged 8-wave one of mfma_wide.hpp).
 #include "decode_util.hpp"

@@ -12,14 +12,15 @@
 // without knowing the routing.  Row groups are the fastest index: an expert's
 // workgroups then go round the 8 XCDs (with 128 slots fastest, each expert
 // had its XCD and a crowded one kept it busy alone: 48 tokens, 46 of them in
-// one expert, 237 -> 139 us; equally popular experts 177 -> 172 us at 32).  (The T <= 8 fused block is moe_block_decode.hip.)
+// one expert, 237 -> 139 us; equally popular experts 177 -> 172 us at 32).
+// (The T <= 8 fused block is moe_block_decode.hip.)
 #include "decode_util.hpp"
 #include "mfma_pipe.hpp"
 
 namespace qmoe {
 
 // ================================================================== gate/up
-// Workgroup: 8 intermediate units (i0 = 8*blockIdx.y); wave w: units i0+2w,
+// Workgroup: 8 intermediate units (i0 = 8*blockIdx.x); wave w: units i0+2w,
 // i0+2w+1 = 2 gate rows + the 2 matching up rows of the packed w13, all in
 // registers (whole 1 KB row pieces per load, requested at once).  The
 // expert's tokens pass over them GU_TOK_CHUNK at a time: wave w copies token
@@ -105,7 +106,7 @@ __global__ __launch_bounds__(256) void moe_gateup_gemv_kernel(
 
 // ================================================================== down
 // Workgroup: (active-expert slot, 64 output columns); wave w owns the 16
-// columns h = 64*blockIdx.y + 16*w + l%16 and computes, on
+// columns h = 64*blockIdx.x + 16*w + l%16 and computes, on
 // v_mfma_f32_16x16x32_bf16, y[token][h] for up to 16 of the expert's tokens
 // at a time:
 //   A (16 x 32): the tokens' fp32 SwiGLU activations as two bf16 parts,

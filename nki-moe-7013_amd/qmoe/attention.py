@@ -25,7 +25,7 @@ def rope_tables(head_dim: int, max_pos: int, theta: float, device) -> tuple:
     return freqs.cos().contiguous(), freqs.sin().contiguous()
 
 
-# Decode batches of up to this many rows take the skinny projection GEMM into
+# Decode batches of up to this many rows project with the plain GEMM into
 # fp32 and finish q/k/v inside the attention launch.
 FUSED_DECODE_MAX_ROWS = 64
 

@@ -23,10 +23,19 @@ import torch
 from . import _lib, ops
 
 # Token counts at or below this use the HBM-bound GEMV experts; above it the
-# MFMA grouped GEMM.  (Each touched expert is streamed once either way.  With
-# 128 equally popular experts the GEMV form is ahead, 190 against 213 us at
-# T = 48 and 193 against 216 us at 64; where a few experts hold most tokens
-# the grouped one is, 116 against 136 us at 48 and 137 against 164 us at 64.)
+# MFMA grouped GEMM.  Each touched expert is streamed once either way; what
+# decides is the largest expert's rows, which the host does not know.  A block
+# of 128 experts in us, GEMV / grouped, by popularity (a router bias of -s
+# log(1 + rank)):
+#   tokens     24           40           48           64
+#   s = 0      169 / 182    200 / 213    207 / 226    214 / 238
+#   s = 0.4    141 / 172    171 / 193    182 / 212    201 / 225
+#   s = 0.8    106 / 126    139 / 137    152 / 145    179 / 148
+#   s = 1.2     95 /  87    123 / 101    137 / 106    169 / 114
+# One token count suits no two of these: GEMVs stay ahead to 64 and past it for
+# equal to moderately skewed experts, to about 40 at s = 0.8 and to fewer than
+# 24 at 1.2.  At 48 the wrong side costs up to 5% at s = 0.8 and 29% at 1.2 below
+# the line, and 11 to 14% at s <= 0.4 above it.
 GEMV_MAX_TOKENS = 48
 # Row tile of the prefill dispatch table: one (up to) 256 x 256 MFMA tile per
 # (tile, panel).
