@@ -305,7 +305,10 @@ __device__ __forceinline__ void down_tile(const TileJob& job, const uint16_t* ac
 // 229).  With several tiles the later ones find the panel in L2, and a
 // non-temporal read of it by the remainder tile cost the full tiles theirs
 // (4096 tokens over 128 equally popular experts: 440 -> 470 us), as did
-// non-temporal half lines on the 32-column stages.
+// non-temporal half lines on the 32-column stages.  Small models alone, whose
+// touched experts stay in the 256 MB Infinity Cache from one token to the next,
+// lose by it (49 tokens of skewed routing over three layers of H = I = 512, 85
+// MB of experts each: 26.5 -> 29.2 us; over ten layers 28.9 -> 27.8).
 template <bool DEVICE>
 __device__ __forceinline__ void gateup_item(const TileJob& job, const uint16_t* __restrict__ x,
                                             const uint16_t* __restrict__ w13, const int32_t* __restrict__ slot_token,
